@@ -36,7 +36,7 @@ LIBRARY = PACKAGE / "kernels" / "libqwen_fused.so"
 PHASES_LIBRARY = PACKAGE / "kernels" / "libqwen_fused_phases.so"
 PHASES_SOURCE = "decode_attention.hip"
 SOURCES = ("rmsnorm.hip", "silu_mul.hip", "qk_norm_rope.hip", "embedding.hip", "skinny_gemm.hip",
-           "decode_attention.hip", "prefill_attention.hip", "row_gemv.hip")
+           "stream_gemm.hip", "decode_attention.hip", "prefill_attention.hip", "row_gemv.hip")
 ARCH = "gfx950"
 
 COMPILE_FLAGS = [

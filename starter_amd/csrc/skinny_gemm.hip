@@ -19,21 +19,23 @@
 // whole 128-byte line at a time.  So W moves in 64-wide k chunks: one
 // 16-byte load per lane reads 8 rows x 128 contiguous bytes (two loads per
 // 16-row tile), the wave writes the chunk to its own LDS staging tile
-// (XOR-swizzled, conflict-free both ways) and reads it back in MFMA layout.  Only the wave itself touches its staging tile, so no
-// workgroup barrier is needed in the loop.  Each wave keeps D chunks of loads
-// in flight (software pipelined).
+// (XOR-swizzled, conflict-free both ways) and reads it back in MFMA layout.
+// Only the wave itself touches its staging tile, so no workgroup barrier is
+// needed in the loop.  Each wave keeps D chunks of loads in flight (software
+// pipelined).
 //
 // A workgroup owns NT n-tiles and one K range (its split); its four waves
 // take interleaved chunks of that range, so together they read consecutive
 // bytes of every row, and reduce their f32 tiles through LDS in wave order.
-// Rows of x beyond M are never stored.
+// Rows of x beyond M are never stored.  This kernel serves up to 16 rows of
+// x; more (and gate/up and the LM head from 5 rows) go to stream_gemm.hip.
 //
 // Two epilogues, as in the reference:
 //   * qf_linear_partials: the workgroup's f32 tile is split `split`'s partial
 //     [S, M, N]; the consumers (qf_add_rms_norm, qf_qkv_norm_rope_cache) add
 //     the S partials in order and round once to bf16.  No atomics, no extra
 //     reduction launch.
-//   * qf_linear_silu_mul: the workgroup owns gate rows [c, c+16h) and the
+//   * qf_linear_silu_mul: the workgroup owns gate rows [c, c+8) and the
 //     matching up rows [N + c, ...) of the packed [2N, K] weight over all of
 //     K, and writes bf16(bf16(silu(bf16(gate))) * bf16(up)).
 //
@@ -48,24 +50,13 @@
 #include "qf_device.h"
 #include "qf_merge.h"
 #include "qf_silu.h"
+#include "qf_skinny.h"
 
 namespace qf {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kTile = 16;    // rows of W (output columns) per n-tile; rows of x per m-tile
-constexpr int kStep = 32;    // k per MFMA
-constexpr int kChunk = 64;   // k per wave chunk; the shape rule's k granularity
 constexpr int kWaves = kBlock / kWave;
-constexpr int kMaxRows = 64;
 constexpr int kColAlign = 32;  // N granularity of the shape rule
-
-// Epilogues.
-constexpr int kEpiPartials = 0;  // f32 split-K partials [S, M, N]
-constexpr int kEpiSiluMul = 1;   // packed gate/up -> bf16 silu(gate) * up [M, N]
-constexpr int kEpiArgmax = 2;    // bf16 logits (optional) + argmax candidates per 16-column tile
 
 // Sources of x in skinny_kernel.
 constexpr int kXDirect = 0;  // global loads straight into MFMA layout (up to 4 rows)
@@ -73,46 +64,6 @@ constexpr int kXStaged = 1;  // loaded like W, transposed through the wave's LDS
 constexpr int kXMerged = 2;  // merged from attention segments into LDS by a prologue
 constexpr int kXNormed = 3;  // RMSNorm of the residual stream, into LDS by a prologue
 constexpr int kNormRows = 4; // most rows kXNormed takes (f64 sums of squares per thread)
-
-// Is (v, i) ahead of (bv, bi) in argmax order: larger value, NaN above
-// everything, the lower index on equal values (torch.argmax's first maximum)?
-__device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
-  const bool vn = v != v, bn = bv != bv;
-  if (vn || bn) return vn && (!bn || i < bi);
-  return v > bv || (v == bv && i < bi);
-}
-
-struct SkinnyArgs {
-  const uint16_t* x;   // [m, k]
-  const uint16_t* w;   // [n, k], or [2n, k] gate rows then up rows
-  float* partials;     // [splits, m, n]; argmax: (value, index) pairs [m, workgroups]
-  uint16_t* out;       // [m, n] (argmax: optional bf16 logits, may be null)
-  int64_t k;
-  int32_t m;
-  int32_t n;           // output columns
-  int32_t chunks;      // 64-wide k chunks per split
-  int32_t splits_major; // 1: blockIdx.x is the split and blockIdx.y the column block
-  // kXMerged only: x row m, columns [128 h, 128 h + 128), is the merge of the
-  // attention segments of virtual head m * seg_kv_heads + h / seg_groups,
-  // query group h % seg_groups (partials [V, S, G, 128], stats [V, S, 2, G]).
-  const float* seg_partials;
-  const float* seg_stats;
-  int32_t seg_splits;
-  int32_t seg_groups;
-  int32_t seg_kv_heads;
-  // kXNormed only: x (the residual stream `total`, bf16 [m, k]) enters as
-  //   inv = 1 / sqrt(f32(sum_g sq[m][g]) / k + eps),  bf16(bf16(x * inv) * gain)
-  // with sq f64 [m, QF_ROW_GROUPS] (per-workgroup sums of squares from
-  // qf_linear_residual) and gain bf16 [k].
-  const double* sq;
-  const uint16_t* gain;
-  float eps;
-};
-
-__device__ __forceinline__ f32x4 mfma(const uint4& a, const uint4& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
 
 // Staging tiles: 128-byte rows, 16-byte piece c of row r stored at piece
 // c ^ ((r >> 1) & 7).  Both access patterns then touch 16 distinct 16-byte
@@ -126,149 +77,99 @@ __device__ __forceinline__ int lds_off(int row, int chunk) {
 }
 constexpr int kRowsPerLoad = kWave * 16 / (kChunk * 2);  // 8 rows x 128 B per load
 
-// Wave hand-off and epilogue shared by the kernel variants: waves wk > 0 of
-// each n-tile group pass their f32 tiles through LDS to wave wk = 0, which
-// adds them in wave order and writes the partials, the SiLU * up product or
-// the argmax candidates.  Called by every wave of the workgroup.
-template <int MT, int NT, int WK, int EPI>
-__device__ __forceinline__ void finish(const SkinnyArgs& a, f32x4 (&acc)[NT][MT], uint8_t* lds,
-                                       int lane, int wk, int wn, int col0, bool live, int split) {
-  constexpr bool PAIRS = EPI == kEpiSiluMul;
-  constexpr bool HALF = PAIRS && NT == 1;  // one tile: 8 gate rows over 8 up rows
-  constexpr int kCols = PAIRS ? NT / 2 : NT;
+// Wave hand-off and epilogue: waves wk > 0 pass their f32 tiles through LDS
+// to wave 0, which adds them in wave order and writes the partials, the SiLU
+// * up product or the argmax candidates.  Called by every wave of the
+// workgroup.
+template <int NT, int EPI>
+__device__ __forceinline__ void finish(const SkinnyArgs& a, f32x4 (&acc)[NT], uint8_t* lds,
+                                       int lane, int wk, int col0, int split) {
   const int r = lane % kTile;
   const int g = lane / kTile;
-  // Waves wk = 1..WK-1 of each group hand their tiles to the group's wave
-  // wk = 0, which adds them in wave order.
-  if constexpr (WK > 1) {
-    __syncthreads();
-    f32x4* handoff = reinterpret_cast<f32x4*>(lds);
-    constexpr int kPer = NT * MT * kWave;
-    if (wk > 0) {
+  __syncthreads();
+  f32x4* handoff = reinterpret_cast<f32x4*>(lds);
+  constexpr int kPer = NT * kWave;
+  if (wk > 0) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          handoff[(wn * (WK - 1) + wk - 1) * kPer + (t * MT + mt) * kWave + lane] = acc[t][mt];
-    }
-    __syncthreads();
-    if (wk > 0) return;
-#pragma unroll
-    for (int w = 0; w < WK - 1; ++w)
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          acc[t][mt] += handoff[(wn * (WK - 1) + w) * kPer + (t * MT + mt) * kWave + lane];
+    for (int t = 0; t < NT; ++t) handoff[(wk - 1) * kPer + t * kWave + lane] = acc[t];
   }
+  __syncthreads();
+  if (wk > 0) return;
+#pragma unroll
+  for (int w = 0; w < kWaves - 1; ++w)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] += handoff[w * kPer + t * kWave + lane];
 
+  const bool row_ok = r < a.m;
   if constexpr (EPI == kEpiArgmax) {
-    // bf16 logits of this wave's 16*NT columns; per row and 16-column tile
-    // the largest, lowest column on ties (NaN counts as largest), reduced
-    // over the four lanes that hold a row of the tile (all lanes take part in
-    // the shuffles); one candidate per row and tile.
+    // bf16 logits of this workgroup's 16*NT columns; per row and 16-column
+    // tile the largest, lowest column on ties (NaN counts as largest),
+    // reduced over the four lanes that hold a row of the tile (all lanes take
+    // part in the shuffles); one candidate per row and tile.
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = kTile * mt + r;
-      const bool row_ok = live && m < a.m;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        float best = -__builtin_inff();
-        int besti = INT32_MAX;
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          v[i] = from_bf16(to_bf16(acc[t][mt][i]));
-          const int col = col0 + kTile * t + 4 * g + i;
-          if (better(v[i], col, best, besti)) {
-            best = v[i];
-            besti = col;
-          }
-        }
-        if (row_ok && a.out)
-          *reinterpret_cast<uint2*>(a.out + (int64_t)m * a.n + col0 + kTile * t + 4 * g) =
-              make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
-#pragma unroll
-        for (int mask = 16; mask <= 32; mask *= 2) {
-          const float ov = __shfl_xor(best, mask);
-          const int oi = __shfl_xor(besti, mask);
-          if (better(ov, oi, best, besti)) {
-            best = ov;
-            besti = oi;
-          }
-        }
-        if (row_ok && g == 0) {
-          uint2* cand = reinterpret_cast<uint2*>(a.partials) + (int64_t)m * (a.n / kTile) +
-                        col0 / kTile + t;
-          *cand = make_uint2(__float_as_uint(best), (uint32_t)besti);
-        }
-      }
-    }
-    return;
-  }
-  if (!live) return;
-  if constexpr (!PAIRS) {
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = kTile * mt + r;
-      if (m >= a.m) continue;
-      float* dst = a.partials + ((int64_t)split * a.m + m) * a.n + col0 + 4 * g;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(dst + kTile * t) = acc[t][mt];
-    }
-  } else if constexpr (HALF) {
-    // Lanes of groups g = 0, 1 hold gate columns col0 + 4g .. +4; groups
-    // 2, 3 the matching up columns, fetched across the wave's halves.
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      float up[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) up[i] = __shfl_xor(acc[0][mt][i], 32);
-      const int m = kTile * mt + r;
-      if (g >= 2 || m >= a.m) continue;
-      float y[4];
+    for (int t = 0; t < NT; ++t) {
+      float best = -__builtin_inff();
+      int besti = INT32_MAX;
+      float v[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float gate = from_bf16(to_bf16(acc[0][mt][i]));
-        y[i] = from_bf16(to_bf16(silu_f32(gate))) * from_bf16(to_bf16(up[i]));
-      }
-      *reinterpret_cast<uint2*>(a.out + (int64_t)m * a.n + col0 + 4 * g) =
-          make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
-    }
-  } else {
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = kTile * mt + r;
-      if (m >= a.m) continue;
-      uint16_t* dst = a.out + (int64_t)m * a.n + col0 + 4 * g;
-#pragma unroll
-      for (int h = 0; h < kCols; ++h) {
-        float y[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          // Each projection is a bf16 tensor in the reference; SiLU is
-          // rounded to bf16 before the bf16 product.
-          const float gate = from_bf16(to_bf16(acc[h][mt][i]));
-          const float up = from_bf16(to_bf16(acc[kCols + h][mt][i]));
-          y[i] = from_bf16(to_bf16(silu_f32(gate))) * up;
+        v[i] = from_bf16(to_bf16(acc[t][i]));
+        const int col = col0 + kTile * t + 4 * g + i;
+        if (better(v[i], col, best, besti)) {
+          best = v[i];
+          besti = col;
         }
-        *reinterpret_cast<uint2*>(dst + kTile * h) = make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
+      }
+      if (row_ok && a.out)
+        *reinterpret_cast<uint2*>(a.out + (int64_t)r * a.n + col0 + kTile * t + 4 * g) =
+            make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+#pragma unroll
+      for (int mask = 16; mask <= 32; mask *= 2) {
+        const float ov = __shfl_xor(best, mask);
+        const int oi = __shfl_xor(besti, mask);
+        if (better(ov, oi, best, besti)) {
+          best = ov;
+          besti = oi;
+        }
+      }
+      if (row_ok && g == 0) {
+        uint2* cand = reinterpret_cast<uint2*>(a.partials) + (int64_t)r * (a.n / kTile) +
+                      col0 / kTile + t;
+        *cand = make_uint2(__float_as_uint(best), (uint32_t)besti);
       }
     }
+  } else if constexpr (EPI == kEpiPartials) {
+    if (!row_ok) return;
+    float* dst = a.partials + ((int64_t)split * a.m + r) * a.n + col0 + 4 * g;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(dst + kTile * t) = acc[t];
+  } else {
+    // Lanes of groups g = 0, 1 hold gate columns col0 + 4g .. +4; groups 2, 3
+    // the matching up columns, fetched across the wave's halves.  Each
+    // projection is a bf16 tensor in the reference; SiLU is rounded to bf16
+    // before the bf16 product.
+    float up[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) up[i] = __shfl_xor(acc[0][i], 32);
+    if (g >= 2 || !row_ok) return;
+    float y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float gate = from_bf16(to_bf16(acc[0][i]));
+      y[i] = from_bf16(to_bf16(silu_f32(gate))) * from_bf16(to_bf16(up[i]));
+    }
+    *reinterpret_cast<uint2*>(a.out + (int64_t)r * a.n + col0 + 4 * g) =
+        make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
   }
 }
 
-// MT m-tiles of x (M <= 16*MT); NT n-tiles of W per wave (for PAIRS the
-// first NT/2 are gate tiles, the rest the matching up tiles; a single PAIRS
-// tile holds 8 gate rows over the matching 8 up rows, its two 8-row loads
-// taken from the two halves of the weight); the four waves
-// form WN = 4/WK groups of distinct n-tiles, each group WK waves that split
-// the chunks; D chunks in flight per wave; NTL = nontemporal weight loads;
-// XS = source of x (kXDirect, kXStaged, kXMerged, kXNormed).  Waves of
-// different groups read the same x chunk at about the same time, so x is
-// fetched from L2 once per workgroup rather than once per wave.
+// One m-tile of x (M <= 16) and NT n-tiles of W per workgroup (gate/up: one
+// tile of 8 gate rows over the matching 8 up rows, its two 8-row loads taken
+// from the two halves of the weight), every wave all of them over its own
+// chunks; D chunks in flight per wave; NTL = nontemporal weight loads; XS =
+// source of x (kXDirect, kXStaged, kXMerged, kXNormed).
 //
-// kXMerged (MT = 1): the workgroup's x slice, M rows x (chunks * 64)
+// kXMerged: the workgroup's x slice, M rows x (chunks * 64)
 // columns = whole heads of the attention output, is merged from the
 // attention segments by the workgroup itself into dynamic LDS (row stride
 // chunks * 128 + 16 bytes), one wave per (row, head), after the first D
@@ -279,23 +180,19 @@ __device__ __forceinline__ void finish(const SkinnyArgs& a, f32x4 (&acc)[NT][MT]
 // 16-byte pieces per thread.  MFMA operands and their order are those of
 // kXDirect: a normalised x equal to qf_add_rms_norm's output gives the bits
 // of qf_linear_partials / qf_linear_silu_mul on it.
-template <int MT, int NT, int WK, int D, int EPI, bool NTL, int XS, int PPT = 0>
+template <int NT, int D, int EPI, bool NTL, int XS, int PPT = 0>
 __global__ __launch_bounds__(kBlock) void skinny_kernel(SkinnyArgs a) {
-  constexpr bool PAIRS = EPI == kEpiSiluMul;
-  constexpr bool HALF = PAIRS && NT == 1;
+  constexpr bool HALF = EPI == kEpiSiluMul;
   constexpr bool XT = XS == kXStaged;
   constexpr bool XM = XS == kXMerged;
   constexpr bool XN = XS == kXNormed;
   constexpr bool XL = XM || XN;  // x read from the prologue's LDS slice
-  static_assert(kWaves % WK == 0, "wave split");
-  static_assert(!XL || MT == 1, "an LDS x slice holds at most 16 rows");
+  static_assert(!HALF || NT == 1, "gate/up: one half tile");
   static_assert(!XN || (kBlock == QF_ROW_GROUPS && PPT >= 1), "normed x: one sum per thread and row");
-  constexpr int WN = kWaves / WK;
-  constexpr int kCols = PAIRS ? NT / 2 : NT;  // output n-tiles per wave
-  constexpr int kColW = HALF ? kTile / 2 : kTile * kCols;  // output columns per wave
-  constexpr int kStageTiles = NT + (XT ? MT : 0);
+  constexpr int kColW = HALF ? kTile / 2 : kTile * NT;  // output columns
+  constexpr int kStageTiles = NT + (XT ? 1 : 0);
   constexpr int kStageBytes = kWaves * kStageTiles * kTileLds;
-  constexpr int kHandoffBytes = WN * (WK - 1) * NT * MT * kWave * 16;
+  constexpr int kHandoffBytes = (kWaves - 1) * NT * kWave * 16;
   __shared__ __attribute__((aligned(16)))
       uint8_t lds[kStageBytes > kHandoffBytes ? kStageBytes : kHandoffBytes];
   extern __shared__ __attribute__((aligned(16))) uint8_t xm_lds[];
@@ -305,10 +202,7 @@ __global__ __launch_bounds__(kBlock) void skinny_kernel(SkinnyArgs a) {
   const int wave = threadIdx.x / kWave;
   const int r = lane % kTile;
   const int g = lane / kTile;
-  const int wk = wave % WK;  // position among the waves sharing n-tiles
-  const int wn = wave / WK;  // n-tile group
-  const int col0 = ((a.splits_major ? blockIdx.y : blockIdx.x) * WN + wn) * kColW;
-  const bool live = col0 < a.n;  // the last workgroup's groups may lie past N
+  const int col0 = (a.splits_major ? blockIdx.y : blockIdx.x) * kColW;
   const int split = a.splits_major ? blockIdx.x : blockIdx.y;
   const int64_t kbase = (int64_t)split * a.chunks * kChunk;
 
@@ -317,54 +211,44 @@ __global__ __launch_bounds__(kBlock) void skinny_kernel(SkinnyArgs a) {
   // col0 + lane / 8, then the up row n further on).
   const uint16_t* wp[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    int row = col0 + kTile * t;
-    if (PAIRS && !HALF && t >= kCols) row = a.n + col0 + kTile * (t - kCols);
-    wp[t] = a.w + (int64_t)(row + lane / 8) * a.k + kbase + 8 * (lane % 8);
-  }
+  for (int t = 0; t < NT; ++t)
+    wp[t] = a.w + (int64_t)(col0 + kTile * t + lane / 8) * a.k + kbase + 8 * (lane % 8);
   const int64_t wstep = HALF ? (int64_t)a.n * a.k : (int64_t)kRowsPerLoad * a.k;
   // Lanes of x rows beyond M read row 0 instead: the MFMA keeps every
   // output column separate, and those columns are never stored.
-  const uint16_t* xp[MT][2];
+  const uint16_t* xp[2];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      if constexpr (XT) {  // coalesced like W, transposed through LDS
-        const int row = kTile * mt + kRowsPerLoad * i + lane / 8;
-        xp[mt][i] = a.x + (int64_t)(row < a.m ? row : 0) * a.k + kbase + 8 * (lane % 8);
-      } else if constexpr (!XL) {  // straight into MFMA layout
-        const int row = kTile * mt + r;
-        xp[mt][i] = a.x + (int64_t)(row < a.m ? row : 0) * a.k + kbase + 8 * g + kStep * i;
-      }
+  for (int i = 0; i < 2; ++i) {
+    if constexpr (XT) {  // coalesced like W, transposed through LDS
+      const int row = kRowsPerLoad * i + lane / 8;
+      xp[i] = a.x + (int64_t)(row < a.m ? row : 0) * a.k + kbase + 8 * (lane % 8);
+    } else if constexpr (!XL) {  // straight into MFMA layout
+      xp[i] = a.x + (int64_t)(r < a.m ? r : 0) * a.k + kbase + 8 * g + kStep * i;
     }
+  }
   uint8_t* stage = lds + wave * kStageTiles * kTileLds;
   const int wr_off[2] = {lds_off(lane / 8, lane % 8), lds_off(lane / 8 + kRowsPerLoad, lane % 8)};
   const int rd_off[2] = {lds_off(r, g), lds_off(r, g + 4)};
   const int xm_row = a.chunks * kChunk * 2 + 16;
   const int xm_off = (r < a.m ? r : 0) * xm_row + 16 * g;
 
-  f32x4 acc[NT][MT];
+  f32x4 acc[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  uint4 wv[D][NT][2], xv[D][MT][2];
-  // This wave's chunks are wk, wk + WK, ...: n_own of them.
-  const int n_own = live && a.chunks > wk ? (a.chunks - wk + WK - 1) / WK : 0;
+  uint4 wv[D][NT][2], xv[D][2];
+  // This wave's chunks are wave, wave + 4, ...: n_own of them.
+  const int n_own = a.chunks > wave ? (a.chunks - wave + kWaves - 1) / kWaves : 0;
 
   auto issue = [&](int d, int j) {
-    const int64_t off = (int64_t)(wk + WK * j) * kChunk;
+    const int64_t off = (int64_t)(wave + kWaves * j) * kChunk;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int i = 0; i < 2; ++i) wv[d][t][i] = load16<NTL>(wp[t] + off + i * wstep);
     if constexpr (!XL) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) xv[d][mt][i] = load16<false>(xp[mt][i] + off);
+      for (int i = 0; i < 2; ++i) xv[d][i] = load16<false>(xp[i] + off);
     }
   };
   // The normed-x prologue: 16-byte piece p of the slice is row p / per_row,
@@ -472,40 +356,31 @@ __global__ __launch_bounds__(kBlock) void skinny_kernel(SkinnyArgs a) {
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        *reinterpret_cast<uint4*>(stage + t * kTileLds + wr_off[i]) =
-            wv[d][t][i];
+        *reinterpret_cast<uint4*>(stage + t * kTileLds + wr_off[i]) = wv[d][t][i];
     if constexpr (XT) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-          *reinterpret_cast<uint4*>(stage + (NT + mt) * kTileLds + wr_off[i]) =
-              xv[d][mt][i];
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<uint4*>(stage + NT * kTileLds + wr_off[i]) = xv[d][i];
     }
     wave_lds_fence();
-    uint4 fw[NT][2], fx[MT][2];
+    uint4 fw[NT][2], fx[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         fw[t][s] = *reinterpret_cast<const uint4*>(stage + t * kTileLds + rd_off[s]);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        if constexpr (XT)
-          fx[mt][s] = *reinterpret_cast<const uint4*>(stage + (NT + mt) * kTileLds + rd_off[s]);
-        else if constexpr (XL)
-          fx[mt][s] = *reinterpret_cast<const uint4*>(xm_lds + xm_off + (wk + WK * j) * kChunk * 2 + s * kStep * 2);
-        else
-          fx[mt][s] = xv[d][mt][s];
-      }
+      if constexpr (XT)
+        fx[s] = *reinterpret_cast<const uint4*>(stage + NT * kTileLds + rd_off[s]);
+      else if constexpr (XL)
+        fx[s] = *reinterpret_cast<const uint4*>(xm_lds + xm_off + (wave + kWaves * j) * kChunk * 2 + s * kStep * 2);
+      else
+        fx[s] = xv[d][s];
     }
     wave_lds_fence();
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[t][mt] = mfma(fw[t][s], fx[mt][s], acc[t][mt]);
+      for (int t = 0; t < NT; ++t) acc[t] = mfma(fw[t][s], fx[s], acc[t]);
   };
 
   // Software pipeline with D chunks in flight.  The steady-state loop issues
@@ -546,161 +421,7 @@ __global__ __launch_bounds__(kBlock) void skinny_kernel(SkinnyArgs a) {
       if (d < n_own) consume(d, d);
   }
 
-  finish<MT, NT, WK, EPI>(a, acc, lds, lane, wk, wn, col0, live, split);
-}
-
-// Variant for 17..64 rows of x, where re-reading x dominates: with the
-// waves of a workgroup splitting K, every workgroup reads its whole x slice
-// from L2 for only 16*NT output columns.  Here the WN = 4 / WK wave groups
-// take distinct n-tiles of the same chunks, and the workgroup stages each x
-// chunk once, cooperatively and coalesced, in a shared LDS ring of two
-// buffers (one barrier per step: a buffer is rewritten only after every wave
-// has passed the barrier that follows its last read).  A step covers WK
-// chunks, one per wave of a group; W still goes through each wave's private
-// staging tile.  All waves run the same number of steps (chunks % WK == 0);
-// waves whose n-tiles lie past N stream row 0 and store nothing.
-template <int MT, int NT, int WK, int D, int EPI, bool NTL>
-__global__ __launch_bounds__(kBlock) void skinny_xs_kernel(SkinnyArgs a) {
-  constexpr bool PAIRS = EPI == kEpiSiluMul;
-  static_assert(!PAIRS || NT % 2 == 0, "gate/up tiles come in pairs here");
-  static_assert(kWaves % WK == 0, "wave split");
-  constexpr int WN = kWaves / WK;
-  constexpr int kCols = PAIRS ? NT / 2 : NT;
-  constexpr int kRows = kTile * MT;                       // staged x rows (M padded)
-  constexpr int kPieces = WK * kRows * (kChunk * 2 / 16);  // 16-byte pieces per step
-  constexpr int XL = (kPieces + kBlock - 1) / kBlock;      // x loads per thread per step
-  constexpr int kXStep = WK * kRows * kLdsRow;             // one ring buffer
-  constexpr int kWStage = kWaves * NT * kTileLds;
-  constexpr int kStageBytes = 2 * kXStep + kWStage;
-  constexpr int kHandoffBytes = WN * (WK - 1) * NT * MT * kWave * 16;
-  __shared__ __attribute__((aligned(16)))
-      uint8_t lds[kStageBytes > kHandoffBytes ? kStageBytes : kHandoffBytes];
-
-  const int tid = threadIdx.x;
-  const int lane = tid % kWave;
-  const int wave = tid / kWave;
-  const int r = lane % kTile;
-  const int g = lane / kTile;
-  const int wk = wave % WK;
-  const int wn = wave / WK;
-  const int col0 = ((a.splits_major ? blockIdx.y : blockIdx.x) * WN + wn) * (kTile * kCols);
-  const bool live = col0 < a.n;
-  const int split = a.splits_major ? blockIdx.x : blockIdx.y;
-  const int64_t kbase = (int64_t)split * a.chunks * kChunk;
-
-  const uint16_t* wp[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    int row = col0 + kTile * t;
-    if (PAIRS && t >= kCols) row = a.n + col0 + kTile * (t - kCols);
-    if (!live) row = 0;
-    wp[t] = a.w + (int64_t)(row + lane / 8) * a.k + kbase + 8 * (lane % 8);
-  }
-  const int64_t wstep = (int64_t)kRowsPerLoad * a.k;
-
-  // Piece p = tid + 256 i of a step: chunk wk' = p / (8 kRows) of the step,
-  // x row (p / 8) % kRows (row 0 stands in for rows past M), 16 bytes at
-  // column 8 * (p % 8) of the chunk.
-  const uint16_t* xp[XL];
-  int xoff[XL];
-  bool xon[XL];
-#pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    const int p = tid + kBlock * i;
-    xon[i] = p < kPieces;
-    const int pc = xon[i] ? p : 0;
-    const int wkp = pc / (8 * kRows);
-    const int row = (pc / 8) % kRows;
-    xp[i] = a.x + (int64_t)(row < a.m ? row : 0) * a.k + kbase + (int64_t)wkp * kChunk + 8 * (pc % 8);
-    xoff[i] = lds_off(wkp * kRows + row, pc % 8);
-  }
-  uint8_t* xring = lds;
-  uint8_t* stage = lds + 2 * kXStep + wave * NT * kTileLds;
-  const int wr_off[2] = {lds_off(lane / 8, lane % 8), lds_off(lane / 8 + kRowsPerLoad, lane % 8)};
-  const int rd_off[2] = {lds_off(r, g), lds_off(r, g + 4)};
-  const int xrd_base = wk * kRows * kLdsRow;  // rows of a multiple of 16 keep the swizzle
-
-  f32x4 acc[NT][MT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  uint4 wv[D][NT][2], xv[D][XL];
-  const int steps = a.chunks / WK;  // the same for every wave
-
-  auto issue = [&](int d, int j) {
-    const int64_t off = (int64_t)(wk + WK * j) * kChunk;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) wv[d][t][i] = load16<NTL>(wp[t] + off + i * wstep);
-    const int64_t xstep = (int64_t)WK * j * kChunk;
-#pragma unroll
-    for (int i = 0; i < XL; ++i) xv[d][i] = xon[i] ? load16<false>(xp[i] + xstep) : make_uint4(0, 0, 0, 0);
-  };
-  auto consume = [&](int d, int j) {
-    uint8_t* xb = xring + (j & 1) * kXStep;
-#pragma unroll
-    for (int i = 0; i < XL; ++i)
-      if (xon[i]) *reinterpret_cast<uint4*>(xb + xoff[i]) = xv[d][i];
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        *reinterpret_cast<uint4*>(stage + t * kTileLds + wr_off[i]) =
-            wv[d][t][i];
-    __syncthreads();
-    uint4 fw[NT][2], fx[MT][2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        fw[t][s] = *reinterpret_cast<const uint4*>(stage + t * kTileLds + rd_off[s]);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        fx[mt][s] = *reinterpret_cast<const uint4*>(xb + xrd_base + mt * kTileLds + rd_off[s]);
-    }
-    wave_lds_fence();
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[t][mt] = mfma(fw[t][s], fx[mt][s], acc[t][mt]);
-  };
-
-  // The same software pipeline as skinny_kernel, D steps in flight.
-  if (steps >= D) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) issue(d, d);
-    int j = 0;
-    for (; j + 2 * D <= steps; j += D) {
-#pragma unroll
-      for (int d = 0; d < D; ++d) {
-        consume(d, j + d);
-        issue(d, j + d + D);
-      }
-    }
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      consume(d, j + d);
-      if (j + d + D < steps) issue(d, j + d + D);
-    }
-    j += D;
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-      if (j + d < steps) consume(d, j + d);
-  } else {
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-      if (d < steps) issue(d, d);
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-      if (d < steps) consume(d, d);
-  }
-
-  finish<MT, NT, WK, EPI>(a, acc, lds, lane, wk, wn, col0, live, split);
+  finish<NT, EPI>(a, acc, lds, lane, wave, col0, split);
 }
 
 // ---- launch plans -----------------------------------------------------------
@@ -712,31 +433,14 @@ int shape_status(int64_t rows, int64_t k, int64_t n) {
   return QF_OK;
 }
 
-// Shared-x wave layout for 17..64 rows (measured on the Qwen3-4B shapes at
-// M = 32 and 64 over tile widths 1-4, wave splits and split counts): each
-// wave all of its workgroup's K range (WK = 1), four steps in flight, and two
-// n-tiles per wave (128 columns per workgroup, half the x re-reads of one)
-// while the grid stays within one workgroup per CU, else one tile.  A CU
-// keeps a bounded number of L1 misses in flight, so the stream needs the
-// workgroups spread over all CUs more than it needs the fewest x re-reads.
-constexpr int64_t kPlanCUs = 256;  // MI355X compute units
-struct XsPlan {
-  int nt, wk, d;
-};
-XsPlan xs_plan(int64_t n, int64_t splits) {
-  const int64_t wide = (n + 8 * kTile - 1) / (8 * kTile) * splits;
-  return wide <= kPlanCUs ? XsPlan{2, 1, 4} : XsPlan{1, 1, 4};
-}
-
 // Power-of-two K splits (measured on the Qwen3-4B projection shapes).  Up to
 // 16 rows: as many as keep every wave at least one chunk, the grid at most
 // 3072 workgroups of 16 columns (~12 per CU), and the partials (written here,
 // read by the consumer) small: splits * min(M, 16) <= K / 32, at most 8 (o_proj
 // takes the same time at 8 and 16 splits, and its consumer, one workgroup per
-// row, reads half the bytes).  Beyond 16 rows (shared-x kernel): K ranges
-// of at most 512 (eight chunks) per workgroup, the fewest splits that give
-// them (Qwen3-4B: qkv 5, o_proj 8, down 19 splits; 10-17% faster at 32 and
-// 64 rows than ~150 workgroups of longer ranges, consumers included).
+// row, reads half the bytes).  Beyond 16 rows: K ranges of at most 512 (eight
+// chunks) per workgroup, the fewest splits that give them (Qwen3-4B: qkv 5,
+// o_proj 8, down 19 splits).
 int plan_splits(int64_t rows, int64_t k, int64_t n) {
   const int64_t chunks = k / kChunk;
   const int64_t mrows = rows < kTile ? rows : kTile;
@@ -764,16 +468,12 @@ dim3 skinny_grid(SkinnyArgs& a, int64_t grid_x, int splits) {
                         : dim3((unsigned)grid_x, (unsigned)splits);
 }
 
-template <int MT, int NT, int WK, int D, int EPI, bool NTL, int XS, int PPT = 0>
+template <int NT, int D, int EPI, bool NTL, int XS, int PPT = 0>
 int launch(const SkinnyArgs& args, int splits, hipStream_t s, size_t dyn_lds = 0) {
-  constexpr bool PAIRS = EPI == kEpiSiluMul;
-  constexpr int kColsPerBlock =
-      (PAIRS && NT == 1 ? kTile / 2 : kTile * (PAIRS ? NT / 2 : NT)) * (kWaves / WK);
+  constexpr int kColsPerBlock = EPI == kEpiSiluMul ? kTile / 2 : kTile * NT;
   SkinnyArgs a = args;
-  const int64_t grid_x = (a.n + kColsPerBlock - 1) / kColsPerBlock;
-  const dim3 grid = skinny_grid(a, grid_x, splits);
-  hipLaunchKernelGGL((skinny_kernel<MT, NT, WK, D, EPI, NTL, XS, PPT>), grid, dim3(kBlock),
-                     dyn_lds, s, a);
+  const dim3 grid = skinny_grid(a, a.n / kColsPerBlock, splits);
+  hipLaunchKernelGGL((skinny_kernel<NT, D, EPI, NTL, XS, PPT>), grid, dim3(kBlock), dyn_lds, s, a);
   return launch_status();
 }
 
@@ -785,73 +485,40 @@ int launch_normed(const SkinnyArgs& a, int splits, hipStream_t s) {
   const int64_t pieces = (int64_t)a.m * a.chunks * (kChunk / 8);
   const size_t lds = (size_t)a.m * (size_t)(a.chunks * kChunk * 2 + 16);
   switch ((pieces + kBlock - 1) / kBlock) {
-    case 1: return launch<1, 1, 4, D, EPI, true, kXNormed, 1>(a, splits, s, lds);
-    case 2: return launch<1, 1, 4, D, EPI, true, kXNormed, 2>(a, splits, s, lds);
-    case 3: return launch<1, 1, 4, D, EPI, true, kXNormed, 3>(a, splits, s, lds);
-    case 4: return launch<1, 1, 4, D, EPI, true, kXNormed, 4>(a, splits, s, lds);
-    case 5: return launch<1, 1, 4, D, EPI, true, kXNormed, 5>(a, splits, s, lds);
+    case 1: return launch<1, D, EPI, true, kXNormed, 1>(a, splits, s, lds);
+    case 2: return launch<1, D, EPI, true, kXNormed, 2>(a, splits, s, lds);
+    case 3: return launch<1, D, EPI, true, kXNormed, 3>(a, splits, s, lds);
+    case 4: return launch<1, D, EPI, true, kXNormed, 4>(a, splits, s, lds);
+    case 5: return launch<1, D, EPI, true, kXNormed, 5>(a, splits, s, lds);
     default: return QF_E_SHAPE;
   }
 }
 
-template <int MT, int NT, int WK, int D, int EPI>
-int launch_xs(const SkinnyArgs& args, int splits, hipStream_t s) {
-  constexpr int kColsPerBlock = kTile * (EPI == kEpiSiluMul ? NT / 2 : NT) * (kWaves / WK);
-  SkinnyArgs a = args;
-  const int64_t grid_x = (a.n + kColsPerBlock - 1) / kColsPerBlock;
-  const dim3 grid = skinny_grid(a, grid_x, splits);
-  hipLaunchKernelGGL((skinny_xs_kernel<MT, NT, WK, D, EPI, true>), grid, dim3(kBlock), 0, s, a);
-  return launch_status();
-}
-
-template <int MT>
-int dispatch_xs_partials(const SkinnyArgs& a, const XsPlan& p, int splits, hipStream_t s) {
-  if (p.nt == 2) return launch_xs<MT, 2, 1, 4, kEpiPartials>(a, splits, s);
-  return launch_xs<MT, 1, 1, 4, kEpiPartials>(a, splits, s);
-}
-
 // Tile plans (measured): up to 4 rows of x arrive as one broadcast line per
 // load, so x goes straight into MFMA layout; up to 16 x is loaded like W and
-// transposed through LDS by each wave; beyond 16 rows the shared-x kernel
-// stages each x chunk once per workgroup (the plain kernel remains for
-// splits whose chunk count does not divide into the plan's steps).
+// transposed through LDS by each wave (the addition order of
+// qf_linear_partials_merged, whose bits these rows share); beyond 16 rows one
+// weight stream per CU (Qwen3-4B at 64 rows against 128-column workgroups
+// staging x per 64 k: qkv 11.0 -> 10.5 us, o_proj 8.9 -> 7.8, down 16.3 ->
+// 14.0; at 17 rows 8.7 -> 8.9, 7.1 -> 6.3, 11.6 -> 11.9).
 int dispatch_partials(const SkinnyArgs& a, int splits, hipStream_t s) {
-  const int mt = (a.m + kTile - 1) / kTile;
-  if (mt > 1) {
-    const XsPlan p = xs_plan(a.n, splits);
-    if (a.chunks % p.wk == 0) {
-      if (mt == 2) return dispatch_xs_partials<2>(a, p, splits, s);
-      if (mt == 3) return dispatch_xs_partials<3>(a, p, splits, s);
-      return dispatch_xs_partials<4>(a, p, splits, s);
-    }
-  }
-  switch (mt) {
-    case 1:
-      if (a.m <= 4) return launch<1, 1, 4, 2, kEpiPartials, true, kXDirect>(a, splits, s);
-      if (a.n / kTile >= 256) return launch<1, 2, 4, 2, kEpiPartials, true, kXStaged>(a, splits, s);
-      return launch<1, 1, 4, 2, kEpiPartials, true, kXStaged>(a, splits, s);
-    case 2: return launch<2, 2, 4, 2, kEpiPartials, true, kXStaged>(a, splits, s);
-    case 3: return launch<3, 2, 4, 2, kEpiPartials, true, kXStaged>(a, splits, s);
-    default: return launch<4, 2, 4, 2, kEpiPartials, true, kXStaged>(a, splits, s);
-  }
+  if (a.m > kTile) return stream_partials(a, splits, s);
+  if (a.m <= 4) return launch<1, 2, kEpiPartials, true, kXDirect>(a, splits, s);
+  if (a.n / kTile >= 256) return launch<2, 2, kEpiPartials, true, kXStaged>(a, splits, s);
+  return launch<1, 2, kEpiPartials, true, kXStaged>(a, splits, s);
 }
 
-// Gate/up + SiLU: all of K per workgroup.  Up to 12 rows one tile of 8 gate
-// over 8 up rows per workgroup (1,216 workgroups for Qwen3-4B: 10% faster at
-// 1-4 rows than a gate and an up tile per wave, whose 608 larger workgroups
-// leave the stream's end unbalanced, 4% at 9-10 rows, even at 12-14, 1%
-// slower at 16; same bits); 13..16 rows the tile pair; beyond 16 rows one
-// gate and one up tile per wave, four waves sharing each staged x chunk.
+// Gate/up + SiLU: all of K per workgroup.  Up to 4 rows one tile of 8 gate
+// over 8 up rows per workgroup (1,216 workgroups for Qwen3-4B: 10% faster
+// than a gate and an up tile per wave, whose 608 larger workgroups leave the
+// stream's end unbalanced; the addition order of the normalising form, whose
+// bits these rows share); beyond, one weight stream per CU (Qwen3-4B against
+// such tiles with x staged per wave at 5 and 16 rows, 20.1 -> 18.7 and 21.7 ->
+// 18.9 us, and against 128-column workgroups at 17 and 64, 23.6 -> 19.4 and
+// 30.6 -> 23.9).
 int dispatch_silu(const SkinnyArgs& a, hipStream_t s) {
-  switch ((a.m + kTile - 1) / kTile) {
-    case 1:
-      if (a.m <= 4) return launch<1, 1, 4, 4, kEpiSiluMul, true, kXDirect>(a, 1, s);
-      if (a.m <= 12) return launch<1, 1, 4, 4, kEpiSiluMul, true, kXStaged>(a, 1, s);
-      return launch<1, 2, 4, 4, kEpiSiluMul, true, kXStaged>(a, 1, s);
-    case 2: return launch_xs<2, 2, 1, 4, kEpiSiluMul>(a, 1, s);
-    case 3: return launch_xs<3, 2, 1, 4, kEpiSiluMul>(a, 1, s);
-    default: return launch_xs<4, 2, 1, 4, kEpiSiluMul>(a, 1, s);
-  }
+  if (a.m <= 4) return launch<1, 4, kEpiSiluMul, true, kXDirect>(a, 1, s);
+  return stream_silu(a, s);
 }
 
 // Final argmax over a row's candidates: one 1024-thread workgroup per row,
@@ -921,34 +588,14 @@ __global__ __launch_bounds__(kFinThreads) void argmax_finalize_kernel(const uint
   }
 }
 
-// LM head plans (measured on the Qwen3-4B head, 151936 x 2560, at 1, 4, 8,
-// 16, 32 and 64 rows): up to 4 rows x straight into MFMA layout with four
-// chunks in flight (two n-tiles per wave from 2 rows); 5..16 rows the
-// shared-x kernel with two n-tiles per wave and wave pairs splitting K (20%
-// faster at 16 rows than per-wave x staging); beyond 16 rows two n-tiles
-// per wave, each wave all of K (10% faster at 32 rows and 18% at 64 than one
-// tile: every workgroup re-reads x, so wider workgroups halve that traffic).
-// Two-tile plans need vocab % 32 == 0.
+// LM head plans (measured on the Qwen3-4B head, 151936 x 2560): up to 4 rows
+// (x as broadcast lines) one 16-column tile per workgroup, the most
+// workgroups; beyond, one weight stream per CU, whose wide column blocks
+// re-read x twice per CU instead of once per 128 columns (8 rows 129.2 ->
+// 125.9 us, 16 134.8 -> 124.9, 32 143.3 -> 130.5, 64 159.6 -> 140.7).
 int dispatch_argmax(const SkinnyArgs& a, hipStream_t s) {
-  const bool two = a.n % (2 * kTile) == 0;
-  switch ((a.m + kTile - 1) / kTile) {
-    case 1:
-      // Up to 4 rows (x as broadcast lines): one 16-column tile per
-      // workgroup, the most workgroups (Qwen3-4B head at 2 and 3 rows: 117.8
-      // -> 114.8 and 118.3 -> 115.7 us against two tiles; even at 4).
-      if (a.m <= 4) return launch<1, 1, 4, 4, kEpiArgmax, true, kXDirect>(a, 1, s);
-      if (!two) return launch_xs<1, 1, 1, 4, kEpiArgmax>(a, 1, s);
-      // 5-16 rows share each staged x chunk among the waves: 32 columns per
-      // workgroup (two wave groups of one tile) up to 8 rows, 128 (four
-      // groups of two) beyond, where x's re-reads weigh more (measured on
-      // the Qwen3-4B head against 64 columns: 122.6 -> 119.1 us at 5 rows,
-      // 124.5 -> 122.3 at 8, 129.0 -> 126.0 at 16).
-      if (a.m <= 8) return launch_xs<1, 1, 2, 4, kEpiArgmax>(a, 1, s);
-      return launch_xs<1, 2, 1, 4, kEpiArgmax>(a, 1, s);
-    case 2: return two ? launch_xs<2, 2, 1, 4, kEpiArgmax>(a, 1, s) : launch_xs<2, 1, 1, 4, kEpiArgmax>(a, 1, s);
-    case 3: return two ? launch_xs<3, 2, 1, 4, kEpiArgmax>(a, 1, s) : launch_xs<3, 1, 1, 4, kEpiArgmax>(a, 1, s);
-    default: return two ? launch_xs<4, 2, 1, 4, kEpiArgmax>(a, 1, s) : launch_xs<4, 1, 1, 4, kEpiArgmax>(a, 1, s);
-  }
+  if (a.m <= 4) return launch<1, 4, kEpiArgmax, true, kXDirect>(a, 1, s);
+  return stream_argmax(a, s);
 }
 
 }  // namespace
@@ -1149,7 +796,7 @@ extern "C" int qf_linear_partials_merged(const float* seg_partials, const float*
   // The same tile plan (and so the same f32 addition order) as
   // qf_linear_partials for up to 16 rows: one 16-row x tile, four waves
   // splitting each workgroup's chunks, two chunks in flight.
-  return launch<1, 1, 4, 2, kEpiPartials, true, kXMerged>(a, splits, as_stream(stream), lds);
+  return launch<1, 2, kEpiPartials, true, kXMerged>(a, splits, as_stream(stream), lds);
 }
 
 namespace qf {

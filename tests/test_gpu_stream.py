@@ -1,0 +1,67 @@
+"""The one-workgroup-per-CU weight streams (partials beyond 16 rows, gate/up and
+LM head from 5) at the edges of their plans: fewer tiles than CUs, one tile
+more than an even share, several column blocks per workgroup, and K ranges of
+one chunk, an odd number of chunks and fewer chunks than the ring holds.
+
+Integer inputs: every partial sum is a whole number below 2^24, so the result
+is exact in any order and compared bit for bit with a float64 product.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from conftest import O, assert_bits_exact, bits, gen
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(), reason="needs an MI355X")]
+
+from starter_amd.kernels import _lib, skinny_gemm as sk  # noqa: E402
+from starter_amd.kernels.lm_head import lm_head_argmax  # noqa: E402
+
+DEV = "cuda"
+
+
+def ints(shape, lo, hi, g):
+    return torch.randint(lo, hi + 1, shape, generator=g).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("m", [17, 32, 33, 48, 64])
+# 2 tiles | 257 shares of 256 | 24 tiles a workgroup (two blocks), K of 1, 3, 5 and 2 chunks a split
+@pytest.mark.parametrize("n,k,splits", [(32, 64, 1), (32, 192, 3), (4128, 192, 1), (6144, 128, 1),
+                                        (2048, 320, 5), (416, 640, 2)])
+def test_partials(m, n, k, splits):
+    g = gen(700 + m + n)
+    x, w = ints((m, k), -4, 4, g), ints((n, k), -3, 3, g)
+    xd, wd = x.to(DEV), w.to(DEV)
+    got = torch.full((splits, m, n), float("nan"), device=DEV)
+    _lib.call("qf_linear_partials", xd.data_ptr(), m, k, wd.data_ptr(), n, splits, got.data_ptr(),
+              _lib.stream(xd.device))
+    per = k // splits
+    want = torch.stack([x.double()[:, s * per:(s + 1) * per] @ w.double()[:, s * per:(s + 1) * per].T
+                        for s in range(splits)]).float()
+    assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("m", [5, 16, 17, 33, 64])
+# 4 half tiles | 260 for 256 workgroups | 20 a workgroup (two blocks)
+@pytest.mark.parametrize("n,k", [(32, 64), (2080, 192), (40960, 64), (96, 1024)])
+def test_silu_mul(m, n, k):
+    g = gen(720 + m + n)
+    x, w = ints((m, k), -2, 2, g), ints((2 * n, k), -1, 1, g)
+    got = sk.linear_silu_mul(x.to(DEV), w.to(DEV))
+    proj = (x.double() @ w.double().T).float().to(torch.bfloat16)
+    assert_bits_exact(got, O.silu_mul(bits(proj)), what=f"silu m={m} n={n} k={k}")
+
+
+@pytest.mark.parametrize("m", [5, 16, 17, 33, 64])
+# 1 tile | 257 tiles for 256 workgroups | 39 a workgroup (three blocks)
+@pytest.mark.parametrize("vocab,k", [(16, 64), (4112, 192), (159760, 64)])
+def test_lm_head(m, vocab, k):
+    g = gen(740 + m + vocab)
+    x, w = ints((m, k), -1, 1, g), ints((vocab, k), -1, 1, g)
+    tokens, logits = lm_head_argmax(x.to(DEV), w.to(DEV), logits=True)
+    want = (x.double() @ w.double().T).float().to(torch.bfloat16)
+    assert torch.equal(logits.cpu(), want)
+    assert torch.equal(tokens.cpu(), want.float().argmax(-1))  # full of ties: the first maximum
