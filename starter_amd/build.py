@@ -22,10 +22,12 @@ Run ``python -m starter_amd.build`` or call :func:`build`.
 from __future__ import annotations
 
 import concurrent.futures
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PACKAGE = Path(__file__).resolve().parent
@@ -35,6 +37,8 @@ OBJ_DIR = PACKAGE / "_build"
 LIBRARY = PACKAGE / "kernels" / "libqwen_fused.so"
 PHASES_LIBRARY = PACKAGE / "kernels" / "libqwen_fused_phases.so"
 PHASES_SOURCE = "decode_attention.hip"
+HOST_CALLS = PACKAGE / "kernels" / "_host_calls.so"
+HOST_SOURCE = "host_calls.cpp"
 SOURCES = ("rmsnorm.hip", "silu_mul.hip", "qk_norm_rope.hip", "embedding.hip", "skinny_gemm.hip",
            "stream_gemm.hip", "decode_attention.hip", "prefill_attention.hip", "row_gemv.hip")
 ARCH = "gfx950"
@@ -67,6 +71,25 @@ def hipcc() -> str:
     return path
 
 
+def _torch_dir() -> Path:
+    return Path(importlib.util.find_spec("torch").origin).parent
+
+
+def _cxx() -> str:
+    return os.environ.get("CXX") or "g++"
+
+
+def _host_flags() -> list[str]:
+    """Flags of the Python extension: torch's and HIP's headers (HIP's want to
+    know the platform when no HIP compiler says it)."""
+    include = _torch_dir() / "include"
+    return ["-O2", "-fPIC", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            "-I", str(ROOT / "include"), "-isystem", str(include),
+            "-isystem", str(include / "torch" / "csrc" / "api" / "include"),
+            "-isystem", str(Path(hipcc()).resolve().parents[1] / "include"),
+            "-isystem", sysconfig.get_paths()["include"]]
+
+
 def _run(cmd: list[str], verbose: bool) -> None:
     if verbose:
         print(" ".join(cmd), flush=True)
@@ -82,7 +105,8 @@ def _run(cmd: list[str], verbose: bool) -> None:
 
 def build(verbose: bool = False) -> Path:
     """Compile every HIP source and link the shared library (and the phase
-    timing library); return the product library's path."""
+    timing library), then the Python extension that calls it
+    (``csrc/host_calls.cpp``, host code only); return the product library's path."""
     cc = hipcc()
     OBJ_DIR.mkdir(exist_ok=True)
     jobs = []
@@ -94,15 +118,23 @@ def build(verbose: bool = False) -> Path:
     phases_job = (phases_obj, [cc, *COMPILE_FLAGS, *EXTRA_FLAGS.get(PHASES_SOURCE, ()),
                                "-DQF_PHASE_STAMPS", "-c", str(CSRC / PHASES_SOURCE),
                                "-o", str(phases_obj)])
-    workers = min(len(jobs) + 1, max(1, min(8, os.cpu_count() or 1)))
+    host_obj = OBJ_DIR / (Path(HOST_SOURCE).stem + ".o")
+    host_job = (host_obj, [_cxx(), *_host_flags(), "-c", str(CSRC / HOST_SOURCE), "-o", str(host_obj)])
+    workers = min(len(jobs) + 2, max(1, min(8, os.cpu_count() or 1)))
     with concurrent.futures.ThreadPoolExecutor(workers) as pool:
-        for fut in [pool.submit(_run, cmd, verbose) for _, cmd in (*jobs, phases_job)]:
+        for fut in [pool.submit(_run, cmd, verbose) for _, cmd in (host_job, *jobs, phases_job)]:
             fut.result()
     for library, objects in ((LIBRARY, [obj for obj, _ in jobs]), (PHASES_LIBRARY, [phases_obj])):
         tmp = library.with_suffix(".so.tmp")
         _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp),
               *[str(obj) for obj in objects]], verbose)
         os.replace(tmp, library)
+    tmp = HOST_CALLS.with_suffix(".so.tmp")
+    torch_lib = _torch_dir() / "lib"
+    _run([_cxx(), "-shared", "-o", str(tmp), str(host_obj), f"-L{LIBRARY.parent}",
+          f"-l:{LIBRARY.name}", "-Wl,-rpath,$ORIGIN", f"-L{torch_lib}", "-lc10", "-lc10_hip",
+          "-ltorch_cpu", "-ltorch_python"], verbose)
+    os.replace(tmp, HOST_CALLS)
     return LIBRARY
 
 

@@ -12,6 +12,7 @@ kernel call raises ``RuntimeError``.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import threading
 from pathlib import Path
 
@@ -93,6 +94,43 @@ def lib() -> ctypes.CDLL:
                     fn.restype = res
                 _handle = handle
     return _handle
+
+
+#: Native forms of the wrappers' ordinary calls (csrc/host_calls.cpp), one call
+#: instead of Python checks, allocations and ctypes conversions: rms_norm
+#: 10.3 -> 5.8 us a call at [8, 2560], linear_partials + run_qkv + linear_partials +
+#: add_rms_norm at 4 x 2081 keys 44.0 -> 27.9 (the GPU work alone).  Each returns NotImplemented, having done
+#: nothing, for any call that it does not take; the wrapper then goes its own
+#: way (checks, errors, strided operands, tensor subclasses, tracing).
+HOST_CALLS = Path(__file__).with_name("_host_calls.so")
+_host = None
+
+
+class _NoHostCalls:
+    """Stands in until the library is built: every call is left to the wrapper."""
+
+    def __getattr__(self, name):
+        return lambda *args: NotImplemented
+
+
+def host():
+    """The native wrappers' module (see HOST_CALLS)."""
+    global _host
+    if _host is None:
+        if not HOST_CALLS.exists():
+            return _NoHostCalls()
+        lib()  # the kernels it calls
+        with _lock:
+            if _host is None:
+                spec = importlib.util.spec_from_file_location("_host_calls", HOST_CALLS)
+                try:
+                    module = importlib.util.module_from_spec(spec)
+                    spec.loader.exec_module(module)
+                except ImportError as error:
+                    raise RuntimeError(f"{HOST_CALLS} does not load ({error}): rebuild it with "
+                                       "`python -m starter_amd.build`") from error
+                _host = module
+    return _host
 
 
 def stream(device: torch.device) -> int:

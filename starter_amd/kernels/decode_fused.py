@@ -59,6 +59,9 @@ def add_rms_norm(residual, branch, weight, eps):
     rounds that sum to bf16 once before the add
     (engine/kernels/decode_fused.py:140-158 is the function this replaces).
     """
+    out = _lib.host().add_rms_norm(residual, branch, weight, eps)
+    if out is not NotImplemented:
+        return out
     n_rows, n_cols = _rows(residual)
     if tuple(weight.shape) != (n_cols,):
         raise ValueError("residual and gain shapes disagree")
@@ -84,6 +87,10 @@ def silu_mul(gate_up, block=1024):
     ``block`` exists so calls written for engine/kernels/decode_fused.py:161
     still bind; the HIP kernel picks its own tiling and ignores it.
     """
+    if type(block) is int and block > 0:
+        out = _lib.host().silu_mul(gate_up)
+        if out is not NotImplemented:
+            return out
     n_rows, width = _rows(gate_up)
     if width % 2:
         raise ValueError("packed gate/up width must be even")
@@ -113,6 +120,10 @@ def qkv_norm_rope_cache(qkv, q_weight, k_weight, q_eps, k_eps, cos, sin, positio
     172-210; unlike it, a position outside [0, capacity) writes nothing and
     the returned Q is all NaN.
     """
+    q = _lib.host().qkv_norm_rope_cache(qkv, q_weight, k_weight, q_eps, k_eps, cos, sin, position,
+                                        key_cache, value_cache)
+    if q is not NotImplemented:
+        return q
     if qkv.ndim == 3 and qkv.dtype == torch.float32:
         if not qkv.is_cuda or not qkv.is_contiguous() or qkv.shape[0] < 1:
             raise ValueError("split-K partials must be contiguous FP32 CUDA [splits, batch, width]")

@@ -35,6 +35,10 @@ def lm_head_argmax(x, weight, logits: bool = False, tokens=None, advance=None):
     int64 [M] tensor on x's device to write the tokens into.  ``advance``:
     optional (position int64 [1], lengths int32 [L]) device tensors that the
     same launches increment by one (the decode step's state advance)."""
+    if tokens is None and advance is None:
+        out = _lib.host().lm_head_argmax(x, weight, logits)
+        if out is not NotImplemented:
+            return out
     if not supports(x, weight):
         raise ValueError("expected contiguous BF16 CUDA x[M<=64,K], W[V,K] with K % 64 == 0, V % 16 == 0")
     rows, k = x.shape

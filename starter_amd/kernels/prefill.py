@@ -32,6 +32,9 @@ def prefill_qkv(qkv, qw, kw, qeps, keps, cos, sin, keys, values, length):
     Returns a new contiguous bf16 Q ``[B, T, Hq, 128]``.  Every tensor on one
     device.  Contract of engine/kernels/prefill.py:66-96.
     """
+    q = _lib.host().prefill_qkv(qkv, qw, kw, qeps, keps, cos, sin, keys, values, length)
+    if q is not NotImplemented:
+        return q
     if keys.ndim != 4 or values.shape != keys.shape:
         raise ValueError("K/V must have matching [B,Hkv,C,D] shapes")
     batch, nk, capacity, width = keys.shape
@@ -65,6 +68,9 @@ def prefill_attention(q, keys, values, length, scale):
     computes this with aten._flash_attention_forward(is_causal=True) on
     ``keys[:, :, :T]`` / ``values[:, :, :T]`` (engine/prefill.py:13-23).
     """
+    out = _lib.host().prefill_attention(q, keys, values, length, scale)
+    if out is not NotImplemented:
+        return out
     if keys.ndim != 4 or values.shape != keys.shape or q.ndim != 4:
         raise ValueError("expected Q [B,T,Hq,D] and K/V caches [B,Hkv,C,D]")
     batch, nk, capacity, width = keys.shape

@@ -58,6 +58,9 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     result is a new contiguous tensor shaped like ``x``
     (engine/kernels/rmsnorm.py:39-62 is the function this replaces).
     """
+    out = _lib.host().rms_norm(x, weight, eps)
+    if out is not NotImplemented:
+        return out
     shape = x.shape
     if x.ndim == 0:
         raise ValueError("rms_norm needs at least one dimension")

@@ -89,6 +89,9 @@ def linear_partials(x, weight):
 
     Mirrors engine/kernels/skinny_gemm.py:100-109.
     """
+    partials = _lib.host().linear_partials(x, weight)
+    if partials is not NotImplemented:
+        return partials
     m, n, k = _dims(x, weight)
     splits = split_count(n, k, m)
     partials = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
@@ -219,6 +222,9 @@ def linear_silu_mul(x, gate_up_weight):
 
     Mirrors engine/kernels/skinny_gemm.py:112-121.
     """
+    out = _lib.host().linear_silu_mul(x, gate_up_weight)
+    if out is not NotImplemented:
+        return out
     m, width, k = _dims(x, gate_up_weight, pairs=True)
     n = width // 2
     out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)

@@ -135,6 +135,12 @@ class SmallQueryAttention:
 
     def _qkv(self, qkv, q_weight, k_weight, q_eps, k_eps, cos, sin, position, key_cache,
              value_cache, used, scale, merge):
+        out = _lib.host().attention_qkv(
+            qkv, q_weight, k_weight, q_eps, k_eps, cos, sin, position, key_cache, value_cache, used,
+            scale, self.partials, self.stats, self.batch, self.hq, self.hk, self.capacity,
+            self.splits, self.span, merge)
+        if out is not NotImplemented:
+            return out
         device = self.partials.device
         width = (self.hq + 2 * self.hk) * HEAD
         if qkv.dtype == torch.float32 and qkv.ndim == 3:
