@@ -111,7 +111,8 @@ struct PrefillArgs {
 // at G = 4, 8 waves of 64 positions (256 rows) need a quarter of the block
 // loads of four 4-wave workgroups of 16.
 // WIDE (8 waves, the ping-pong schedule) is taken when the grid has at least
-// one workgroup per CU (1 x 2048, 4 x 512 and up at Qwen3-4B's heads).
+// one workgroup per CU (1 x 2048, 4 x 512 and up at Qwen3-4B's heads) and the
+// prompt is not a short one (kShortPrompt).
 // Smaller prompts take the 4-wave form, which at G = 4 holds 16 positions
 // per workgroup (one tile per wave, 157 VGPRs: two workgroups per CU; with
 // 32 positions and two tiles per wave it needed 312 registers, one
@@ -130,6 +131,13 @@ template <> struct Split<4, true> { static constexpr int QB = 64, TPW = 2, W = 8
 template <> struct Split<8, false> { static constexpr int QB = 16, TPW = 2, W = 4; };
 template <> struct Split<8, true> { static constexpr int QB = 32, TPW = 2, W = 8; };
 constexpr int64_t kWideWorkgroups = kCUs;
+// Prompts that fill at most three quarters of one 8-wave workgroup of the
+// G = 4 form take the 4-wave form in any number: the wide one would compute
+// 64 positions for each (128 x 5 22.9 -> 8.5 us, 64 x 17 13.5 -> 9.2, 64 x 40
+// 17.5 -> 14.6, 64 x 48 19.5 -> 16.1, 128 x 48 35.4 -> 32.2; 64 x 56 20.9
+// against 20.4, 32 x 64 11.3 against 13.9).  At G = 8, 32 positions wide, the
+// wide form stays ahead (256 x 17 15.0 against 18.9 us).
+constexpr int64_t kShortPrompt = 48;
 
 __device__ __forceinline__ f32x4 mfma32(const uint4& a, const uint4& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
@@ -590,8 +598,8 @@ int launch_prefill_as(PrefillArgs a, hipStream_t s) {
 template <int G>
 int launch_prefill(PrefillArgs a, hipStream_t s) {
   const int64_t wide_blocks = (a.length + Split<G, true>::QB - 1) / Split<G, true>::QB * a.pairs;
-  return wide_blocks >= kWideWorkgroups ? launch_prefill_as<G, true>(a, s)
-                                        : launch_prefill_as<G, false>(a, s);
+  const bool wide = wide_blocks >= kWideWorkgroups && !(G == 4 && a.length <= kShortPrompt);
+  return wide ? launch_prefill_as<G, true>(a, s) : launch_prefill_as<G, false>(a, s);
 }
 
 }  // namespace

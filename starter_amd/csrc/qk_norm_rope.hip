@@ -152,7 +152,7 @@ struct PrefillArgs {
   uint32_t nq, nk;
   uint32_t q_units, k_units, units;  // nq / 8, nk / 8, (nq + 2 nk) / 8
   FastDiv heads;           // nq + 2 nk
-  FastDiv waves_per_token; // ceil(units / kUnitsPerWave)
+  FastDiv waves_per_token; // ceil(units / units per wave)
   FastDiv length;
   const uint16_t* qw;
   const uint16_t* kw;
@@ -169,12 +169,19 @@ struct PrefillArgs {
 // head row: [8l, 8l+8) and their rotate-half partners [64+8l, 64+8l+8), so
 // the partner exchange needs no cross-lane traffic and a row is reduced over
 // 8 lanes (3 DPP steps).  A "unit" is 8 consecutive head rows of one token
-// with one role (q, k or v), one per 8-lane group of a wave.  A wave owns up
-// to kUnitsPerWave consecutive units of one token: its loads all issue first,
+// with one role (q, k or v), one per 8-lane group of a wave.  A wave owns one
+// or two (kUnitsPerWave) consecutive units of one token: its loads all issue first,
 // the token's cos/sin row and both gains are unpacked once per wave, roles
 // are wave-uniform (scalar branches) and v units are pure copies.
 // Qwen3-4B: 6 units per token -> 3 waves of 2 units.
 constexpr int kUnitsPerWave = 2;
+// Calls of at most this many units are latency, not bytes: one unit per wave
+// halves the chain (1 x 17 tokens 3.3 -> 2.6 us, 1 x 128 3.5 -> 2.8, 1 x 512
+// 5.7 -> 5.4; 1 x 1024 7.4 with two units, 8.0 with one).  Below the streaming
+// size workgroups are one wave, which spread over more CUs (1 x 1024 7.8 ->
+// 7.3 us, 16 x 128 11.6 -> 11.3); streaming calls keep four (4 x 2048 34.9
+// against 36.3).
+constexpr uint64_t kSmallUnits = 12 * kCUs;
 constexpr int kRowLanes = 8;  // lanes per head row in the unit kernel
 
 // Norm + gain + RoPE of one head row spread as 16 elements per lane over 8
@@ -217,11 +224,11 @@ __device__ __forceinline__ void norm_rope16(const float* x, const float* w, cons
 // unit loop carry no bounds branch; measured on the Qwen3-4B 4 x 2048 call
 // 34.0 us against 35.2 us with the checks (a copy with this kernel's loads and
 // stores and no arithmetic takes 33.0 us).
-template <bool NT, bool FULL, int UPW = kUnitsPerWave, int MIN_WAVES = 1>
-__global__ __launch_bounds__(kBlock, MIN_WAVES) void prefill_qkv_unit_kernel(PrefillArgs a) {
+template <bool NT, bool FULL, int UPW, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void prefill_qkv_unit_kernel(PrefillArgs a) {
   const uint32_t wave =
-      __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave);
-  if (wave >= a.waves) return;  // wave-uniform
+      __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / kWave) + threadIdx.x / kWave);
+  if (BLOCK > kWave && wave >= a.waves) return;  // wave-uniform
   const uint32_t token = __builtin_amdgcn_readfirstlane(fdiv(wave, a.waves_per_token));
   const uint32_t first =
       __builtin_amdgcn_readfirstlane((wave - token * a.waves_per_token.d) * UPW);
@@ -440,25 +447,22 @@ extern "C" int qf_prefill_qkv(const void* qkv, int64_t batch, int64_t length, in
     a.q_units = (uint32_t)nq / kRowLanes;
     a.k_units = (uint32_t)nk / kRowLanes;
     a.units = (uint32_t)heads / kRowLanes;
-    const uint32_t per_token = (a.units + kUnitsPerWave - 1) / kUnitsPerWave;
+    const bool stream = (int64_t)rows * kD * 4 >= kStreamBytes;
+    const uint32_t upw = tokens * a.units <= kSmallUnits ? 1 : kUnitsPerWave;
+    const uint32_t per_token = (a.units + upw - 1) / upw;
     a.waves_per_token = make_fastdiv(per_token);
     const uint64_t waves = tokens * per_token;
     a.waves = (uint32_t)waves;
-    const uint64_t blocks = (waves + kBlock / kWave - 1) / (kBlock / kWave);
-    const bool stream = (int64_t)rows * kD * 4 >= kStreamBytes;
-    const bool full = a.units % kUnitsPerWave == 0;
-    if (stream && full)
-      hipLaunchKernelGGL((prefill_qkv_unit_kernel<true, true>), dim3((unsigned)blocks),
-                         dim3(kBlock), 0, s, a);
-    else if (stream)
-      hipLaunchKernelGGL((prefill_qkv_unit_kernel<true, false>), dim3((unsigned)blocks),
-                         dim3(kBlock), 0, s, a);
-    else if (full)
-      hipLaunchKernelGGL((prefill_qkv_unit_kernel<false, true>), dim3((unsigned)blocks),
-                         dim3(kBlock), 0, s, a);
-    else
-      hipLaunchKernelGGL((prefill_qkv_unit_kernel<false, false>), dim3((unsigned)blocks),
-                         dim3(kBlock), 0, s, a);
+    const bool full = a.units % upw == 0;
+    const dim3 wide((unsigned)((waves + kBlock / kWave - 1) / (kBlock / kWave))), narrow((unsigned)waves);
+#define QF_UNITS(NT, FULL, UPW, BLOCK, GRID) \
+  hipLaunchKernelGGL((prefill_qkv_unit_kernel<NT, FULL, UPW, BLOCK>), GRID, dim3(BLOCK), 0, s, a)
+    if (upw == 1) QF_UNITS(false, true, 1, kWave, narrow);
+    else if (stream && full) QF_UNITS(true, true, kUnitsPerWave, kBlock, wide);
+    else if (stream) QF_UNITS(true, false, kUnitsPerWave, kBlock, wide);
+    else if (full) QF_UNITS(false, true, kUnitsPerWave, kWave, narrow);
+    else QF_UNITS(false, false, kUnitsPerWave, kWave, narrow);
+#undef QF_UNITS
     return launch_status();
   }
   hipLaunchKernelGGL(prefill_qkv_kernel, dim3(blocks_for(rows)), dim3(kBlock), 0, s, a);
