@@ -4,7 +4,7 @@
   epsilon and calls ``kernels.rmsnorm.rms_norm``.
 * ``PackedMLP`` - engine/mlp.py:8-21: one packed ``[2I, H]`` gate/up weight;
   on CUDA bf16 the activation is the fused ``silu_mul`` kernel on the packed
-  projection, elsewhere it is the reference module's own ``act_fn(gate) * up``.
+  projection (up to 64 rows one launch for both, ``linear_silu_mul``), elsewhere it is the reference module's own ``act_fn(gate) * up``.
 * ``DecodeQKNormRoPE`` - engine/qk_norm_rope.py:10-71: a ``Qwen3Attention``
   whose single-token decode forward runs the per-head Q/K RMSNorm and the
   rotary embedding as one ``kernels.qk_norm_rope`` launch; every other call
@@ -30,6 +30,7 @@ from .kernels.decode_fused import silu_mul
 from .kernels.embedding import FusedEmbedding
 from .kernels.qk_norm_rope import HEAD, qk_norm_rope
 from .kernels.rmsnorm import rms_norm
+from .kernels.skinny_gemm import MAX_ROWS, linear_silu_mul, supports
 
 __all__ = ["FusedRMSNorm", "PackedMLP", "DecodeQKNormRoPE", "FusedEmbedding", "install"]
 
@@ -59,7 +60,25 @@ class PackedMLP(nn.Module):
         self.down_proj = reference.down_proj
         self.act_fn = reference.act_fn
 
+    def _decode_hidden(self, x):
+        """The activation of decode-sized inputs (at most 64 rows) from the
+        gate/up weight stream with its SiLU epilogue, or None where that does
+        not apply.  The library's product reads the same weight at under half
+        its rate there, then writes and re-reads the projections (this module
+        at the Qwen3-4B widths, 1 / 21 / 64 rows: 66.5 -> 38.1 us, 53.6 -> 39.5,
+        62.7 -> 52.3).  64 rows are what the stream kernel's x tiles hold."""
+        if (not x.is_cuda or x.dtype != torch.bfloat16 or x.ndim < 1 or torch.is_autocast_enabled("cuda")
+                or not 1 <= x.numel() // max(x.shape[-1], 1) <= MAX_ROWS or not _is_silu(self.act_fn)):
+            return None
+        rows = x.reshape(-1, x.shape[-1])
+        if not supports(rows, self.gate_up_weight, pairs=True):
+            return None
+        return linear_silu_mul(rows, self.gate_up_weight).view(*x.shape[:-1], -1)
+
     def forward(self, x):
+        hidden = self._decode_hidden(x)
+        if hidden is not None:
+            return self.down_proj(hidden)
         projected = F.linear(x, self.gate_up_weight)
         if projected.is_cuda and projected.dtype == torch.bfloat16 and _is_silu(self.act_fn):
             width = projected.shape[-1]

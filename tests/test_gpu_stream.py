@@ -17,6 +17,7 @@ from conftest import O, assert_bits_exact, bits, gen
 pytestmark = [pytest.mark.gpu,
               pytest.mark.skipif(not torch.cuda.is_available(), reason="needs an MI355X")]
 
+from starter_amd import modules  # noqa: E402
 from starter_amd.kernels import _lib, skinny_gemm as sk  # noqa: E402
 from starter_amd.kernels.lm_head import lm_head_argmax  # noqa: E402
 
@@ -65,3 +66,33 @@ def test_lm_head(m, vocab, k):
     want = (x.double() @ w.double().T).float().to(torch.bfloat16)
     assert torch.equal(logits.cpu(), want)
     assert torch.equal(tokens.cpu(), want.float().argmax(-1))  # full of ties: the first maximum
+
+
+class _MLP(torch.nn.Module):
+    def __init__(self, hidden, inner, g):
+        super().__init__()
+        self.gate_proj, self.up_proj = (torch.nn.Linear(hidden, inner, bias=False) for _ in range(2))
+        self.down_proj, self.act_fn = torch.nn.Linear(inner, hidden, bias=False), torch.nn.SiLU()
+        for p in self.parameters():
+            p.data = torch.randn(p.shape, generator=g) * 0.1
+
+
+@pytest.mark.parametrize("shape", [(1, 256), (2, 3, 256), (64, 256), (65, 256), (1, 0, 256)])
+@pytest.mark.parametrize("inner", [320, 96])  # 96: not whole column pairs, the library's product
+@pytest.mark.parametrize("form", ["plain", "strided", "autocast"])
+@torch.no_grad()
+def test_packed_mlp_on_both_sides_of_its_row_rule(shape, inner, form):
+    """The module on decode-sized inputs against the projections and activation in sequence: within
+    the f32 accumulation of a projection, which moves single bf16 values by one rounding."""
+    g = gen(760 + inner)
+    module = modules.PackedMLP(_MLP(256, inner, g).cuda().bfloat16())
+    x = torch.randn(shape, generator=g).cuda().bfloat16()
+    if form == "strided":
+        x = torch.stack([x, x], -1)[..., 0]
+    with torch.autocast("cuda", dtype=torch.float16, enabled=form == "autocast"):
+        got = module(x)
+        projected = torch.nn.functional.linear(x, module.gate_up_weight)
+        gate, up = projected.chunk(2, -1)
+        want = module.down_proj(torch.nn.functional.silu(gate) * up)
+    assert got.shape == want.shape and got.dtype == want.dtype
+    torch.testing.assert_close(got.float(), want.float(), rtol=0.02, atol=0.02 * float(want.float().abs().max()) if want.numel() else 0)
