@@ -110,34 +110,33 @@ struct PrefillArgs {
 // G * QB query rows, so its K/V traffic from L2 per flop falls as that grows:
 // at G = 4, 8 waves of 64 positions (256 rows) need a quarter of the block
 // loads of four 4-wave workgroups of 16.
-// WIDE (8 waves, the ping-pong schedule) is taken when the grid has at least
-// one workgroup per CU (1 x 2048, 4 x 512 and up at Qwen3-4B's heads) and the
-// prompt is not a short one (kShortPrompt).
-// Smaller prompts take the 4-wave form, which at G = 4 holds 16 positions
-// per workgroup (one tile per wave, 157 VGPRs: two workgroups per CU; with
-// 32 positions and two tiles per wave it needed 312 registers, one
-// workgroup per CU) - four times the 8-wave form's workgroups, each with a
-// shorter chain per key block.  Measured (Qwen3-4B heads, bit-identical
-// outputs): 1 x 512 18.7 -> 13.4 us, 2 x 512 19.3 -> 15.5, 3 x 512 20.5 ->
-// 18.7, 1 x 1024 32.3 -> 24.4, 1 x 1536 45.7 -> 34.6 against 32 positions;
-// the 8-wave form stays ahead from one workgroup per CU (1 x 2048 53.9
-// against 57.1 us, 4 x 512 21.2 against 21.9) and behind below it (1 x 1024
-// 30.8, 3 x 512 20.5 at 128 and 192 workgroups).
-template <int G, bool WIDE> struct Split;
-template <bool WIDE> struct Split<1, WIDE> { static constexpr int QB = 64, TPW = 1, W = 4; };
-template <bool WIDE> struct Split<2, WIDE> { static constexpr int QB = 64, TPW = 2, W = 4; };
-template <> struct Split<4, false> { static constexpr int QB = 16, TPW = 1, W = 4; };
-template <> struct Split<4, true> { static constexpr int QB = 64, TPW = 2, W = 8; };
-template <> struct Split<8, false> { static constexpr int QB = 16, TPW = 2, W = 4; };
-template <> struct Split<8, true> { static constexpr int QB = 32, TPW = 2, W = 8; };
-constexpr int64_t kWideWorkgroups = kCUs;
-// Prompts that fill at most three quarters of one 8-wave workgroup of the
-// G = 4 form take the 4-wave form in any number: the wide one would compute
-// 64 positions for each (128 x 5 22.9 -> 8.5 us, 64 x 17 13.5 -> 9.2, 64 x 40
-// 17.5 -> 14.6, 64 x 48 19.5 -> 16.1, 128 x 48 35.4 -> 32.2; 64 x 56 20.9
-// against 20.4, 32 x 64 11.3 against 13.9).  At G = 8, 32 positions wide, the
-// wide form stays ahead (256 x 17 15.0 against 18.9 us).
-constexpr int64_t kShortPrompt = 48;
+//
+// kNarrow: one tile per wave (two workgroups per CU where LDS allows) on the
+// single-wave pipeline: the most workgroups and the shortest chain per key
+// block, for grids that do not fill the chip.  kMid and kWide: 8 waves on the
+// ping-pong schedule, one and two tiles per wave (G = 2: one, 64 positions).
+// All forms give the same bits.  Measured (Qwen3-4B heads, us, narrow / mid /
+// wide): 1 x 512 13.4 / - / 18.7, 1 x 1024 23.2 / 36.9 / 30.0, 8 x 128 8.3 / 8.4 /
+// 10.8, 16 x 128 13.4 / 12.7 / 12.9, 64 x 17 10.5 / 8.3 / 14.3, 64 x 64 20.8 /
+// 19.2 / 22.5, 64 x 160 52.6 / 44.9 / 57.4, 64 x 256 113 / 96.6 / 93.1, 16 x 333
+// 41.0 / 36.4 / 39.1, 16 x 512 75.7 / 64.6 / 57.0; 16 over 8 heads (narrow /
+// wide): 16 x 333 24.7 / 26.5, 16 x 512 41.8 / 39.6, 4 x 2048 106 / 93.9, 1 x
+// 4096 102 / 134; 16 over 2 (mid / wide) 256 x 24 15.4 / 17.6, 256 x 64 37.4 /
+// 42.4, 4 x 2048 95.6 / 75.7.  Earlier shapes: two tiles per wave in the narrow
+// form at G = 2 (1 x 333 13.4 -> 9.9, 1 x 2048 54.8 -> 43.9) and 8 (1 x 333
+// 13.5 -> 11.0), no ping-pong at G = 2 (4 x 2048 117.9 -> 93.9).
+constexpr int kNarrow = 0, kMid = 1, kWide = 2;
+template <int G, int FORM> struct Split;
+template <int FORM> struct Split<1, FORM> { static constexpr int QB = 64, TPW = 1, W = 4; };
+template <> struct Split<2, kNarrow> { static constexpr int QB = 32, TPW = 1, W = 4; };
+template <> struct Split<2, kWide> { static constexpr int QB = 64, TPW = 1, W = 8; };
+template <> struct Split<4, kNarrow> { static constexpr int QB = 16, TPW = 1, W = 4; };
+template <> struct Split<4, kMid> { static constexpr int QB = 32, TPW = 1, W = 8; };
+template <> struct Split<4, kWide> { static constexpr int QB = 64, TPW = 2, W = 8; };
+template <> struct Split<8, kNarrow> { static constexpr int QB = 16, TPW = 1, W = 8; };
+template <> struct Split<8, kMid> { static constexpr int QB = 16, TPW = 1, W = 8; };
+template <> struct Split<8, kWide> { static constexpr int QB = 32, TPW = 2, W = 8; };
+template <int G, int FORM> constexpr bool ping_pong() { return FORM != kNarrow && Split<G, FORM>::W == 8; }
 
 __device__ __forceinline__ f32x4 mfma32(const uint4& a, const uint4& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
@@ -149,11 +148,11 @@ __device__ __forceinline__ v4i16 read_tr(const uint8_t* base, int off) {
       (lds_v4i16*)((__attribute__((address_space(3))) uint8_t*)base + off));
 }
 
-template <int G, bool WIDE>
-__global__ __launch_bounds__((Split<G, WIDE>::W * kWave)) void prefill_attn_kernel(PrefillArgs a) {
-  constexpr int QB = Split<G, WIDE>::QB;
-  constexpr int TPW = Split<G, WIDE>::TPW;
-  constexpr int W = Split<G, WIDE>::W;
+template <int G, int FORM>
+__global__ __launch_bounds__((Split<G, FORM>::W * kWave)) void prefill_attn_kernel(PrefillArgs a) {
+  constexpr int QB = Split<G, FORM>::QB;
+  constexpr int TPW = Split<G, FORM>::TPW;
+  constexpr int W = Split<G, FORM>::W;
   constexpr int kSubs = QB / 16;  // position tiles per head
   constexpr int kKLoads = kKB * kKRow / 1024;  // 1 KB direct loads per staged K block (17)
   constexpr int kVLoads = kKB * kVRow / 1024;  // ... per V block (18)
@@ -421,7 +420,7 @@ __global__ __launch_bounds__((Split<G, WIDE>::W * kWave)) void prefill_attn_kern
 
   const int dtn = (int)((pt + 15 - (int64_t)(nkb - 1) * kKB) >> 4) + 1;  // diagonal tiles, 1..4
   const int dks = dtn > 2 ? 2 : 1;
-  if constexpr (W == 8) {
+  if constexpr (ping_pong<G, FORM>()) {
     // Ping-pong between the two waves of each SIMD: waves 0-3 and 4-7 run
     // the same steps, the second set one step behind, so that while one wave
     // of a SIMD issues matrix-core products (step M j: block j - 1's P V,
@@ -541,7 +540,7 @@ __global__ __launch_bounds__((Split<G, WIDE>::W * kWave)) void prefill_attn_kern
   // O / l in bf16 through LDS (this wave's 16 x 128 tile; lane l writes the
   // 8 bytes of dims 16 db + 4 g4 .. + 3 of its own query), read back so that
   // every lane stores 16 contiguous bytes of one output row.
-  if constexpr (W != 8) __syncthreads();  // every wave is done with the K blocks
+  if constexpr (!ping_pong<G, FORM>()) __syncthreads();  // every wave is done with the K blocks
   uint8_t* ot = reinterpret_cast<uint8_t*>(klds) + wave * 16 * kORow;  // both K buffers
 #pragma unroll
   for (int u = 0; u < TPW; ++u) {
@@ -583,23 +582,35 @@ int32_t work_group(int32_t pairs, int32_t qblocks) {
   return g < per_xcd ? g : 0;
 }
 
-template <int G, bool WIDE>
-int launch_prefill_as(PrefillArgs a, hipStream_t s) {
-  constexpr int QB = Split<G, WIDE>::QB;
+template <int G, int FORM>
+int launch_prefill_as(PrefillArgs a, bool ordered, hipStream_t s) {
+  constexpr int QB = Split<G, FORM>::QB;
   a.qblocks = (int32_t)((a.length + QB - 1) / QB);
   const int64_t blocks = (int64_t)a.qblocks * a.pairs;
   if (blocks > (int64_t)INT32_MAX) return QF_E_SHAPE;
-  a.group = WIDE ? work_group(a.pairs, a.qblocks) : 0;
-  hipLaunchKernelGGL((prefill_attn_kernel<G, WIDE>), dim3((unsigned)blocks),
-                     dim3(Split<G, WIDE>::W * kWave), 0, s, a);
+  a.group = ordered ? work_group(a.pairs, a.qblocks) : 0;
+  hipLaunchKernelGGL((prefill_attn_kernel<G, FORM>), dim3((unsigned)blocks),
+                     dim3(Split<G, FORM>::W * kWave), 0, s, a);
   return launch_status();
 }
 
+// The wide form takes grids that fill the chip: one of its workgroups per CU,
+// four at G = 2 (one tile per wave there, so a narrow workgroup costs a
+// quarter of its).  Of those, prompts that its positions per workgroup fit
+// badly take the mid form, half as wide: under four wide blocks of positions,
+// or up to six blocks with the last at most half full; the shortest of all
+// take 16 positions.
 template <int G>
 int launch_prefill(PrefillArgs a, hipStream_t s) {
-  const int64_t wide_blocks = (a.length + Split<G, true>::QB - 1) / Split<G, true>::QB * a.pairs;
-  const bool wide = wide_blocks >= kWideWorkgroups && !(G == 4 && a.length <= kShortPrompt);
-  return wide ? launch_prefill_as<G, true>(a, s) : launch_prefill_as<G, false>(a, s);
+  constexpr int QB = Split<G, kWide>::QB;
+  const int64_t wide = (a.length + QB - 1) / QB, tail = a.length - (wide - 1) * QB;
+  if (wide * a.pairs < (G == 2 ? 4 : 1) * (int64_t)kCUs)
+    return launch_prefill_as<G, kNarrow>(a, false, s);
+  if constexpr (G >= 4) {
+    if (G == 4 && a.length <= 16) return launch_prefill_as<G, kNarrow>(a, false, s);
+    if (a.length < 4 * QB || (wide <= 6 && tail <= QB / 2)) return launch_prefill_as<G, kMid>(a, true, s);
+  }
+  return launch_prefill_as<G, kWide>(a, true, s);
 }
 
 }  // namespace

@@ -1,6 +1,6 @@
-"""Prompt kernels on both sides of their small-call rules: the attention's
-workgroup form for batches of short prompts, and the Q/K/V kernel's units per
-wave (one up to 3,072 units of 8 head rows, two beyond)."""
+"""Prompt kernels on both sides of their dispatch rules: the attention's
+workgroup forms, and the Q/K/V kernel's units per wave (one up to 3,072 units of
+8 head rows, two beyond)."""
 
 from __future__ import annotations
 
@@ -17,21 +17,41 @@ from starter_amd.kernels.prefill import prefill_attention, prefill_qkv  # noqa: 
 DEV = "cuda"
 
 
-# 33 x 8 pairs: at least one wide workgroup per CU; 48 | 49 positions: 4-wave form | 8-wave form
-@pytest.mark.parametrize("length", [1, 5, 16, 17, 48, 49, 64])
-def test_attention_of_many_short_prompts(length):
-    g = gen(800 + length)
-    batch, hq, hk, capacity = 33, 32, 8, length + 3
-    q, k, v = (normal((batch, n, t, 128), g=g) for n, t in ((length, hq), (hk, capacity), (hk, capacity)))
+def check_attention(batch, length, hq, hk):
+    g = torch.Generator(device=DEV).manual_seed(800 + length + hq)
+    capacity = length + 3
+    q, k, v = (torch.randn(batch, n, t, 128, generator=g, device=DEV).bfloat16()
+               for n, t in ((length, hq), (hk, capacity), (hk, capacity)))
     k[:, :, length:], v[:, :, length:] = float("nan"), float("nan")  # slots past the prompt are never read
-    got = prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), length, 128 ** -0.5).float().cpu()
-    kf, vf = (t[:, :, :length].float().repeat_interleave(hq // hk, 1) for t in (k, v))
-    s = (q.float().transpose(1, 2) @ kf.transpose(2, 3).contiguous()) * 128 ** -0.5
-    s.masked_fill_(torch.ones(length, length).triu(1).bool(), float("-inf"))
-    want = (torch.softmax(s, -1) @ vf).transpose(1, 2)
-    # the bar of the reference's attention tests: bf16 probabilities and output
-    torch.testing.assert_close(got, want, rtol=0.02, atol=0.004 * 4)
-    assert float((got - want).norm() / want.norm()) < 0.01
+    got = prefill_attention(q, k, v, length, 128 ** -0.5).float()
+    hide = torch.ones(length, length, device=DEV).triu(1).bool()
+    for b in range(0, batch, max(1, batch // 5)):
+        kf, vf = (t[b, :, :length].float().repeat_interleave(hq // hk, 0) for t in (k, v))
+        s = (q[b].float().transpose(0, 1) @ kf.transpose(1, 2).contiguous()) * 128 ** -0.5
+        want = (torch.softmax(s.masked_fill(hide, float("-inf")), -1) @ vf).transpose(0, 1)
+        # bf16 probabilities (2^-9 of a sum of up to 4 x |v|) and output (2^-8)
+        torch.testing.assert_close(got[b], want, rtol=0.02, atol=0.016)
+        assert float((got[b] - want).norm() / want.norm()) < 0.01
+
+
+# at least one wide workgroup per CU: 16 | 17 positions, one to four wide blocks, a fifth and a sixth
+# at most and over half full, seven
+@pytest.mark.parametrize("batch,length", [(33, 1), (33, 5), (33, 16), (33, 17), (33, 48), (33, 64), (33, 65), (9, 255),
+                                          (9, 256), (9, 257), (9, 288), (9, 289), (9, 352), (9, 353), (9, 385)])
+def test_attention_forms_at_four_heads_per_kv_head(batch, length):
+    check_attention(batch, length, 32, 8)
+
+
+# 1,023 | 1,024 wide workgroups: the narrow form | the 8-wave form
+@pytest.mark.parametrize("batch,length,hk", [(1, 1, 8), (3, 97, 8), (341, 64, 3), (256, 33, 4), (128, 64, 8), (64, 65, 8)])
+def test_attention_forms_at_two_heads_per_kv_head(batch, length, hk):
+    check_attention(batch, length, 2 * hk, hk)
+
+
+# under | at one wide workgroup per CU; up to four wide blocks of 32, a fifth half full and fuller
+@pytest.mark.parametrize("batch,length", [(1, 1), (5, 130), (128, 3), (128, 33), (64, 127), (64, 128), (64, 144), (64, 145)])
+def test_attention_forms_at_eight_heads_per_kv_head(batch, length):
+    check_attention(batch, length, 16, 2)
 
 
 @pytest.mark.parametrize("batch,length,nq,nk", [(1, 1, 32, 8), (3, 5, 16, 8), (1, 512, 32, 8), (1, 513, 32, 8),
