@@ -17,7 +17,7 @@
 //   D[4*(l/16) + i][l % 16] = y[m0 + l%16][n0 + 4*(l/16) + i].
 //   Waves: MG groups of two m-tiles times 8 / MG groups of n-tiles
 //   (tile t to group t % (8 / MG)); every output has one wave and one chain
-//   of additions in ascending k, so no reduction between waves is needed.
+//   of additions, so no reduction between waves is needed.
 //
 // A ring tile is 16 rows of 256 bytes; 16-byte piece p of row r sits at piece
 // p ^ r, so the 16 lanes of a fragment read touch all 64 banks once.  The DMA
@@ -145,7 +145,13 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
   }
   const uint32_t ring0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)ring +
                          kLoadBytes * q;
-  int is_tile = t_lo, is_stage = 0;                // next stage to issue
+  // Column group c takes the stages of its K range from stage c on, around
+  // the end.  All groups in step would read the same columns of rows a
+  // constant stride apart, and a stride of 4 or 8 KB sends those to few
+  // memory channels (64 rows: K = 2048 LM head 150 -> 113 us, K = 4096 232 ->
+  // 213, gate/up 46.0 -> 38.2; K = 2560 and 3072 even).
+  const int first = group % stages;
+  int is_tile = t_lo, is_step = 0, is_stage = first;  // next stage to issue
   auto issue = [&](int slot) {
     // Past the split's range in a half-filled last stage: re-read its first
     // half (those LDS pieces are not used).
@@ -169,8 +175,9 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
       const int mt = x0 + TG * c;
       if (mt < MT) dma16<false>(xrow[c] + off, dst + (NT + mt) * kTileBytes);
     }
-    if (++is_stage == stages) {
-      is_stage = 0;
+    if (++is_stage == stages) is_stage = 0;
+    if (++is_step == stages) {
+      is_step = 0;
       is_tile += NT;
     }
   };
@@ -279,7 +286,7 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
 #pragma unroll
   for (int d = 0; d < S - 1; ++d)
     if (d < total) issue(d);
-  int slot = 0, next = S - 1, at = 0, tile0 = t_lo;
+  int slot = 0, next = S - 1, at = 0, stage = first, tile0 = t_lo;
   constexpr int kPer = kTiles / TG, kMore = kTiles % TG;  // loads per stage: kPer + (tg < kMore)
   for (int it = 0; it < total; ++it) {
     const int later = total - 1 - it;              // stages after this one, issued or not
@@ -289,15 +296,14 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
     asm volatile("" ::: "memory");
     if (it + S - 1 < total) issue(next);
     const uint8_t* buf = ring + slot * kStageBytes;
+    if (ragged && stage == stages - 1) stage_products(buf, std::integral_constant<int, kChunk / kStep>{});
+    else stage_products(buf, std::integral_constant<int, kSteps>{});
+    stage = stage + 1 == stages ? 0 : stage + 1;
     if (++at == stages) {
-      if (ragged) stage_products(buf, std::integral_constant<int, kChunk / kStep>{});
-      else stage_products(buf, std::integral_constant<int, kSteps>{});
       store(tile0);
       clear();
       at = 0;
       tile0 += NT;
-    } else {
-      stage_products(buf, std::integral_constant<int, kSteps>{});
     }
     slot = slot + 1 == S ? 0 : slot + 1;
     next = next + 1 == S ? 0 : next + 1;
