@@ -499,8 +499,8 @@ int launch_normed(const SkinnyArgs& a, int splits, hipStream_t s) {
 // transposed through LDS by each wave (the addition order of
 // qf_linear_partials_merged, whose bits these rows share); beyond 16 rows one
 // weight stream per CU (Qwen3-4B at 64 rows against 128-column workgroups
-// staging x per 64 k: qkv 11.0 -> 10.5 us, o_proj 8.9 -> 7.8, down 16.3 ->
-// 14.0; at 17 rows 8.7 -> 8.9, 7.1 -> 6.3, 11.6 -> 11.9).
+// staging x per 64 k: qkv 10.6 -> 10.2 us, o_proj 8.4 -> 7.9, down 15.1 ->
+// 13.6; at 17 rows 8.4 -> 8.4, 7.1 -> 6.7, 11.5 -> 11.6).
 int dispatch_partials(const SkinnyArgs& a, int splits, hipStream_t s) {
   if (a.m > kTile) return stream_partials(a, splits, s);
   if (a.m <= 4) return launch<1, 2, kEpiPartials, true, kXDirect>(a, splits, s);

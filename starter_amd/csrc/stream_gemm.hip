@@ -341,15 +341,19 @@ int launch_stream(const SkinnyArgs& s, int splits, hipStream_t stream) {
                        stream, a);                                                     \
     return launch_status();                                                            \
   }
-  // Up to 6 tiles 128 k per stage (256-byte runs of each weight row), wider
-  // blocks 64 k, so that three stages fit the LDS.
+  // Up to 8 tiles 128 k per stage (256-byte runs of each weight row), wider
+  // blocks 64 k, so that three stages fit the LDS (Qwen3-4B qkv, 8 tiles, at
+  // 32 and 64 rows 9.2 -> 8.7 and 10.9 -> 10.2 us with 128; gate/up, 5 tiles, at
+  // 64 rows 27.5 -> 23.9; down and LM head, 13 and 19 tiles, 16.0 -> 13.9 and
+  // 154 -> 140 with 64 and the wider blocks it allows).  More than three stages
+  // in flight measured slower or even.
   QF_STREAM(1, 128)
   QF_STREAM(2, 128)
   QF_STREAM(3, 128)
   QF_STREAM(4, 128)
   QF_STREAM(5, 128)
   QF_STREAM(6, 128)
-  QF_STREAM(8, 64)
+  QF_STREAM(8, 128)
   QF_STREAM(10, 64)
   QF_STREAM(13, 64)
   QF_STREAM(16, 64)
