@@ -419,7 +419,7 @@ int qf_decode_attention_qkv(const void* qkv, int32_t qkv_splits, const void* q_w
                             void* out, void* stream);
 
 /*
- * Candidate slots per row that qf_lm_head_argmax needs (vocab / 16), or a
+ * Candidate slots per row that qf_lm_head_argmax may use (vocab / 16), or a
  * negative status when vocab is not a positive multiple of 16.
  */
 int64_t qf_lm_head_blocks(int64_t vocab);

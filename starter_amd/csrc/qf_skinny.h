@@ -14,7 +14,7 @@ constexpr int kMaxRows = 64;
 // Epilogues.
 constexpr int kEpiPartials = 0;  // f32 split-K partials [S, M, N]
 constexpr int kEpiSiluMul = 1;   // packed gate/up -> bf16 silu(gate) * up [M, N]
-constexpr int kEpiArgmax = 2;    // bf16 logits (optional) + argmax candidates per 16-column tile
+constexpr int kEpiArgmax = 2;    // bf16 logits (optional) + argmax candidates per workgroup
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -58,6 +58,13 @@ struct SkinnyArgs {
   const uint16_t* gain;
   float eps;
 };
+
+// Column groups of a weight stream: one workgroup per CU over all splits
+// (fewer for small outputs).
+inline int32_t stream_groups(int32_t tiles, int splits) {
+  const int fill = kCUs / splits < 1 ? 1 : kCUs / splits;
+  return fill < tiles ? fill : tiles;
+}
 
 // The 17..64-row projections (stream_gemm.hip): x, w, partials / out, k, m, n
 // and chunks set, checked by the caller.

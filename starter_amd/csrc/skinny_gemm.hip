@@ -521,15 +521,16 @@ int dispatch_silu(const SkinnyArgs& a, hipStream_t s) {
   return stream_silu(a, s);
 }
 
-// Final argmax over a row's candidates: one 1024-thread workgroup per row,
-// each thread four candidates in flight per round (9,496 candidates for
-// Qwen3-4B: three rounds instead of 37 loads in turn per thread).  The
+// Final argmax over a row's candidates: one workgroup per row, each thread
+// four candidates in flight per round.  1024 threads for one candidate per 16
+// columns (up to 4 rows; 9,496 for Qwen3-4B: three rounds instead of 37 loads
+// in turn per thread), 256 for one per workgroup of a weight stream.  The
 // order (larger value, NaN largest, then the lower index) is total, so the
 // reduction order does not change the result.
-constexpr int kFinThreads = 1024;
 constexpr int kFinUnroll = 4;
 // With `position` set, workgroup 0 also advances the decode position and
 // the per-head lengths by one (the step's last writes, in the same launch).
+template <int kFinThreads>
 __global__ __launch_bounds__(kFinThreads) void argmax_finalize_kernel(const uint2* cand,
                                                                      int64_t blocks,
                                                                      int64_t* tokens,
@@ -593,8 +594,9 @@ __global__ __launch_bounds__(kFinThreads) void argmax_finalize_kernel(const uint
 // workgroups; beyond, one weight stream per CU, whose wide column blocks
 // re-read x twice per CU instead of once per 128 columns (8 rows 129.2 ->
 // 125.9 us, 16 134.8 -> 124.9, 32 143.3 -> 130.5, 64 159.6 -> 140.7).
+constexpr int kArgmaxTileRows = 4;
 int dispatch_argmax(const SkinnyArgs& a, hipStream_t s) {
-  if (a.m <= 4) return launch<1, 4, kEpiArgmax, true, kXDirect>(a, 1, s);
+  if (a.m <= kArgmaxTileRows) return launch<1, 4, kEpiArgmax, true, kXDirect>(a, 1, s);
   return stream_argmax(a, s);
 }
 
@@ -644,9 +646,14 @@ int lm_head_argmax(const void* x, int64_t rows, int64_t k, const void* weight, i
   hipStream_t s = as_stream(stream);
   const int st = dispatch_argmax(a, s);
   if (st != QF_OK) return st;
-  hipLaunchKernelGGL(argmax_finalize_kernel, dim3((unsigned)rows), dim3(kFinThreads), 0, s,
-                     static_cast<const uint2*>(candidates), vocab / kTile, tokens, position,
-                     lengths, length_count);
+  const uint2* cand = static_cast<const uint2*>(candidates);
+  if (rows <= kArgmaxTileRows)
+    hipLaunchKernelGGL(argmax_finalize_kernel<1024>, dim3((unsigned)rows), dim3(1024), 0, s, cand,
+                       vocab / kTile, tokens, position, lengths, length_count);
+  else
+    hipLaunchKernelGGL(argmax_finalize_kernel<256>, dim3((unsigned)rows), dim3(256), 0, s, cand,
+                       (int64_t)stream_groups(a.n / kTile, 1), tokens, position, lengths,
+                       length_count);
   return launch_status();
 }
 

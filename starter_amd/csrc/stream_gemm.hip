@@ -220,6 +220,13 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
     else products(buf, std::integral_constant<int, NTW - 1>{}, steps_tag);
   };
 
+  float best[MTW];                                 // argmax form only
+  int besti[MTW];
+#pragma unroll
+  for (int j = 0; j < MTW; ++j) {
+    best[j] = -__builtin_inff();
+    besti[j] = INT32_MAX;
+  }
   auto store = [&](int tile0) {
 #pragma unroll
     for (int i = 0; i < NTW; ++i) {
@@ -248,35 +255,23 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
                 make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
           }
         } else {
-          // bf16 logits; per row and tile the largest, lowest column on ties
-          // (NaN largest), over the four lanes that hold a row of the tile.
-          float best = -__builtin_inff(), y[4];
-          int besti = INT32_MAX;
+          // bf16 logits; per lane and row the largest so far, lowest column on
+          // ties (NaN largest).
+          if (live && m < a.m) {
+            float y[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            y[e] = from_bf16(to_bf16(v[e]));
-            const int col = kTile * t + 4 * g + e;
-            if (better(y[e], col, best, besti)) {
-              best = y[e];
-              besti = col;
+            for (int e = 0; e < 4; ++e) {
+              y[e] = from_bf16(to_bf16(v[e]));
+              const int col = kTile * t + 4 * g + e;
+              if (better(y[e], col, best[j], besti[j])) {
+                best[j] = y[e];
+                besti[j] = col;
+              }
             }
+            if (a.out)
+              *reinterpret_cast<uint2*>(a.out + (int64_t)m * a.n + kTile * t + 4 * g) =
+                  make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
           }
-          const bool ok = live && m < a.m;
-          if (ok && a.out)
-            *reinterpret_cast<uint2*>(a.out + (int64_t)m * a.n + kTile * t + 4 * g) =
-                make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
-#pragma unroll
-          for (int mask = 16; mask <= 32; mask *= 2) {
-            const float ov = __shfl_xor(best, mask);
-            const int oi = __shfl_xor(besti, mask);
-            if (better(ov, oi, best, besti)) {
-              best = ov;
-              besti = oi;
-            }
-          }
-          if (ok && g == 0)
-            reinterpret_cast<uint2*>(a.partials)[(int64_t)m * a.tiles + t] =
-                make_uint2(__float_as_uint(best), (uint32_t)besti);
         }
       }
     }
@@ -308,10 +303,45 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
     slot = slot + 1 == S ? 0 : slot + 1;
     next = next + 1 == S ? 0 : next + 1;
   }
+
+  if constexpr (EPI == kEpiArgmax) {
+    // One candidate per row and workgroup: over the four lanes of a row, then,
+    // through the drained ring, over the waves of its m-tile.  (One per 16
+    // columns gave the last kernel 9,496 a row to read, and as many 8-byte
+    // stores: the Qwen3-4B head with logits at 64 rows 147.4 -> 144.9 us.)
+    uint2* cand = reinterpret_cast<uint2*>(ring);  // [NG][MG * MTW * 16 rows]
+    constexpr int kRows = MG * MTW * kTile;
+    __syncthreads();                               // the last stage is read
+#pragma unroll
+    for (int j = 0; j < MTW; ++j) {
+#pragma unroll
+      for (int mask = 16; mask <= 32; mask *= 2) {
+        const float ov = __shfl_xor(best[j], mask);
+        const int oi = __shfl_xor(besti[j], mask);
+        if (better(ov, oi, best[j], besti[j])) {
+          best[j] = ov;
+          besti[j] = oi;
+        }
+      }
+      if (g == 0)
+        cand[wn * kRows + kTile * (wm * MTW + j) + r] =
+            make_uint2(__float_as_uint(best[j]), (uint32_t)besti[j]);
+    }
+    __syncthreads();
+    const int m = threadIdx.x;
+    if (m < a.m) {                                 // a.m <= kRows
+      uint2 top = cand[m];
+#pragma unroll
+      for (int w = 1; w < NG; ++w) {
+        const uint2 c = cand[w * kRows + m];
+        if (better(__uint_as_float(c.x), (int)c.y, __uint_as_float(top.x), (int)top.y)) top = c;
+      }
+      reinterpret_cast<uint2*>(a.partials)[(int64_t)m * a.groups + group] = top;
+    }
+  }
 }
 
-// Column groups: one workgroup per CU over all splits (fewer for small
-// outputs), each an equal run of n-tiles; a block of it is as wide as the
+// Column groups (stream_groups): each an equal run of n-tiles; a block of it is as wide as the
 // ring takes (x is re-read once per block), evenly cut.
 constexpr int kMaxBlockTiles = 19;
 
@@ -328,8 +358,7 @@ int launch_stream(const SkinnyArgs& s, int splits, hipStream_t stream) {
   a.chunks = s.chunks;
   a.splits = splits;
   a.tiles = s.n / (EPI == kEpiSiluMul ? kTile / 2 : kTile);
-  const int fill = kCUs / splits < 1 ? 1 : kCUs / splits;
-  a.groups = fill < a.tiles ? fill : a.tiles;
+  a.groups = stream_groups(a.tiles, splits);
   const int most = (a.tiles + a.groups - 1) / a.groups;          // tiles of a group
   const int blocks = (most + kMaxBlockTiles - 1) / kMaxBlockTiles;
   const int need = (most + blocks - 1) / blocks;                 // tiles of a block

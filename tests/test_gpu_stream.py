@@ -68,6 +68,22 @@ def test_lm_head(m, vocab, k):
     assert torch.equal(tokens.cpu(), want.float().argmax(-1))  # full of ties: the first maximum
 
 
+@pytest.mark.parametrize("m", [5, 33, 64])
+@pytest.mark.parametrize("fill", ["nan", "-inf"])
+def test_lm_head_order_across_workgroups(m, fill):
+    """NaN above everything and the first of several; a row of nothing but -inf picks column 0."""
+    vocab, k = 4112, 64
+    g = gen(750 + m)
+    x, w = torch.ones(m, k).bfloat16(), ints((vocab, k), -1, 1, g)
+    if fill == "nan":
+        w[[4111, 2049, 3000]] = float("nan")
+        w[17] = float("inf")
+    else:
+        w[:] = float("-inf")
+    tokens, _ = lm_head_argmax(x.to(DEV), w.to(DEV), logits=True)
+    assert tokens.tolist() == [2049 if fill == "nan" else 0] * m
+
+
 class _MLP(torch.nn.Module):
     def __init__(self, hidden, inner, g):
         super().__init__()
