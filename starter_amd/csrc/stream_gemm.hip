@@ -91,8 +91,8 @@ __device__ __forceinline__ void wait_stages(int stages) {
   }
 }
 
-// KW: k per ring stage.
-template <int MT, int NT, int KW, int EPI>
+// KW: k per ring stage; PHASED: K in quarters, from a start of the group's own.
+template <int MT, int NT, int KW, int EPI, bool PHASED>
 __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
   constexpr bool PAIRS = EPI == kEpiSiluMul;
   constexpr int MG = MT > 2 ? 2 : 1;               // wave groups over m
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
   const int t_hi = (int)((int64_t)(group + 1) * a.tiles / a.groups);
   const int64_t kbase = (int64_t)split * a.chunks * kChunk;
   const int stages = (a.chunks * kChunk + KW - 1) / KW;
-  const bool ragged = KW > kChunk && (a.chunks & 1);  // last stage half filled
+  const bool ragged = !PHASED && KW > kChunk && (a.chunks & 1);  // last stage half filled
   const int blocks = (t_hi - t_lo + NT - 1) / NT;
   const int total = blocks * stages;
 
@@ -145,13 +145,18 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
   }
   const uint32_t ring0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)ring +
                          kLoadBytes * q;
-  // Column group c takes the stages of its K range from stage c on, around
-  // the end.  All groups in step would read the same columns of rows a
-  // constant stride apart, and a stride of 4 or 8 KB sends those to few
-  // memory channels (64 rows: K = 2048 LM head 150 -> 113 us, K = 4096 232 ->
-  // 213, gate/up 46.0 -> 38.2; K = 2560 and 3072 even).
-  const int first = group % stages;
-  int is_tile = t_lo, is_step = 0, is_stage = first;  // next stage to issue
+  // PHASED: part v of a group's pass over K is quarter v ^ phase, and the
+  // quarters are added as (q0 + q1) + (q2 + q3).  Whatever the phase, the same
+  // sums are formed (with their two sides in either order, which rounds the
+  // same), so a weight row's result does not depend on its group, on N or on
+  // how the columns are sharded.  The phase is hashed so that it does not run
+  // with the group's address bits (16,384-column gate/up at K = 4096, 64 rows:
+  // 77 us with a start that follows the group number, 45 hashed).
+  constexpr int kParts = PHASED ? 4 : 1;
+  const int per_part = stages / kParts;            // PHASED: K is a multiple of 1,024
+  const int phase = PHASED ? (int)(((uint32_t)group * 0x9E3779B1u) >> 30) : 0;
+  // Next stage to issue: stage is_in of part is_part of the block at is_tile.
+  int is_tile = t_lo, is_part = 0, is_in = 0, is_stage = phase * per_part;
   auto issue = [&](int slot) {
     // Past the split's range in a half-filled last stage: re-read its first
     // half (those LDS pieces are not used).
@@ -175,14 +180,20 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
       const int mt = x0 + TG * c;
       if (mt < MT) dma16<false>(xrow[c] + off, dst + (NT + mt) * kTileBytes);
     }
-    if (++is_stage == stages) is_stage = 0;
-    if (++is_step == stages) {
-      is_step = 0;
-      is_tile += NT;
+    ++is_stage;
+    if (++is_in == per_part) {
+      is_in = 0;
+      if (++is_part == kParts) {
+        is_part = 0;
+        is_tile += NT;
+      }
+      is_stage = (is_part ^ phase) * per_part;
     }
   };
 
   f32x4 acc[NTW][MTW];
+  // PHASED: the quarter, and the half, that wait for the other side of their sum.
+  f32x4 quarter[PHASED ? NTW : 1][PHASED ? MTW : 1], half[PHASED ? NTW : 1][PHASED ? MTW : 1];
   auto clear = [&] {
 #pragma unroll
     for (int i = 0; i < NTW; ++i)
@@ -277,13 +288,13 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
     }
   };
 
-  clear();
 #pragma unroll
   for (int d = 0; d < S - 1; ++d)
     if (d < total) issue(d);
-  int slot = 0, next = S - 1, at = 0, stage = first, tile0 = t_lo;
+  int slot = 0, next = S - 1;
   constexpr int kPer = kTiles / TG, kMore = kTiles % TG;  // loads per stage: kPer + (tg < kMore)
-  for (int it = 0; it < total; ++it) {
+  // Stage `it` of the sequence; `last`: the last one of its block.
+  auto step = [&](int it, bool last) {
     const int later = total - 1 - it;              // stages after this one, issued or not
     if (tg < kMore) wait_stages<kPer + 1, S - 2>(later);
     else wait_stages<kPer, S - 2>(later);
@@ -291,17 +302,42 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
     asm volatile("" ::: "memory");
     if (it + S - 1 < total) issue(next);
     const uint8_t* buf = ring + slot * kStageBytes;
-    if (ragged && stage == stages - 1) stage_products(buf, std::integral_constant<int, kChunk / kStep>{});
+    if (ragged && last) stage_products(buf, std::integral_constant<int, kChunk / kStep>{});
     else stage_products(buf, std::integral_constant<int, kSteps>{});
-    stage = stage + 1 == stages ? 0 : stage + 1;
-    if (++at == stages) {
-      store(tile0);
-      clear();
-      at = 0;
-      tile0 += NT;
-    }
     slot = slot + 1 == S ? 0 : slot + 1;
     next = next + 1 == S ? 0 : next + 1;
+  };
+  clear();
+  int tile0 = t_lo;
+  if constexpr (PHASED) {
+    for (int it = 0; it < total; tile0 += NT) {
+#pragma unroll
+      for (int part = 0; part < kParts; ++part) {
+        for (int at = 0; at < per_part; ++at, ++it) step(it, false);
+#pragma unroll
+        for (int i = 0; i < NTW; ++i)
+#pragma unroll
+          for (int j = 0; j < MTW; ++j) {
+            if (part % 2 == 1) acc[i][j] += quarter[i][j];
+            if (part == 3) acc[i][j] += half[i][j];
+            if (part % 2 == 0) quarter[i][j] = acc[i][j];
+            if (part == 1) half[i][j] = acc[i][j];
+          }
+        if (part == 3) store(tile0);
+        clear();
+      }
+    }
+  } else {
+    int at = 0;
+    for (int it = 0; it < total; ++it) {
+      step(it, at == stages - 1);
+      if (++at == stages) {
+        store(tile0);
+        clear();
+        at = 0;
+        tile0 += NT;
+      }
+    }
   }
 
   if constexpr (EPI == kEpiArgmax) {
@@ -343,10 +379,13 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
 
 // Column groups (stream_groups): each an equal run of n-tiles; a block of it is as wide as the
 // ring takes (x is re-read once per block), evenly cut.
-constexpr int kMaxBlockTiles = 19;
+// PHASED beyond 32 rows: 16, where the two held sums still fit the registers
+// (19 spill: the 151,936-column head at K = 2048, 64 rows 159 us, 16 132).
+template <int MT, bool PHASED>
+constexpr int kMaxBlockTiles = PHASED && MT > 2 ? 16 : 19;
 
-template <int MT, int EPI>
-int launch_stream(const SkinnyArgs& s, int splits, hipStream_t stream) {
+template <int MT, int EPI, bool PHASED>
+int launch_stream_as(const SkinnyArgs& s, int splits, hipStream_t stream) {
   StreamArgs a;
   a.x = s.x;
   a.w = s.w;
@@ -360,14 +399,16 @@ int launch_stream(const SkinnyArgs& s, int splits, hipStream_t stream) {
   a.tiles = s.n / (EPI == kEpiSiluMul ? kTile / 2 : kTile);
   a.groups = stream_groups(a.tiles, splits);
   const int most = (a.tiles + a.groups - 1) / a.groups;          // tiles of a group
-  const int blocks = (most + kMaxBlockTiles - 1) / kMaxBlockTiles;
+  constexpr int kMost = kMaxBlockTiles<MT, PHASED>;
+  const int blocks = (most + kMost - 1) / kMost;
   const int need = (most + blocks - 1) / blocks;                 // tiles of a block
   a.splits_major = splits > 1 && s.k >= s.n ? 1 : 0;
   const dim3 grid((unsigned)((int64_t)a.groups * splits));
 #define QF_STREAM(NT, KW)                                                              \
+  if constexpr (NT <= kMost)                                                           \
   if (need <= NT) {                                                                    \
-    hipLaunchKernelGGL((stream_kernel<MT, NT, KW, EPI>), grid, dim3(kStreamBlock), 0,  \
-                       stream, a);                                                     \
+    hipLaunchKernelGGL((stream_kernel<MT, NT, KW, EPI, PHASED>), grid,                 \
+                       dim3(kStreamBlock), 0, stream, a);                              \
     return launch_status();                                                            \
   }
   // Up to 8 tiles 128 k per stage (256-byte runs of each weight row), wider
@@ -389,6 +430,21 @@ int launch_stream(const SkinnyArgs& s, int splits, hipStream_t stream) {
   QF_STREAM(19, 64)
 #undef QF_STREAM
   return QF_E_SHAPE;  // not reached: need <= kMaxBlockTiles
+}
+
+// All workgroups in step read the same columns of rows a constant stride apart,
+// and strides of 2, 4 or 8 KB send those to few memory channels.  So at K a
+// multiple of 1,024 in one range, a quarter of the workgroups starts in each
+// quarter of K (64 rows, in order -> PHASED: 151,936-column head at K = 2048
+// 155 -> 132 us; at K = 1024 73 -> 76, but 130,304 columns 71 -> 62; 12,288-column
+// gate/up at K = 4096 41.8 -> 36.6, at K = 2048 24.0 -> 21.1).  Other strides
+// measured even (K = 2560) and split ranges start apart by themselves: there K
+// goes in order.
+template <int MT, int EPI>
+int launch_stream(const SkinnyArgs& a, int splits, hipStream_t s) {
+  if constexpr (EPI != kEpiPartials)
+    if (a.k % 1024 == 0) return launch_stream_as<MT, EPI, true>(a, splits, s);
+  return launch_stream_as<MT, EPI, false>(a, splits, s);
 }
 
 template <int EPI>

@@ -84,6 +84,26 @@ def test_lm_head_order_across_workgroups(m, fill):
     assert tokens.tolist() == [2049 if fill == "nan" else 0] * m
 
 
+@pytest.mark.parametrize("m", [5, 17, 33, 64])
+# in order (an odd number of chunks, 64 and 128 k per stage) | in quarters
+@pytest.mark.parametrize("k", [320, 2560, 1024, 4096])
+def test_column_bits_do_not_depend_on_their_place(m, k):
+    """Equal weight rows give equal bits wherever they stand, in a call of any width: the order of
+    additions is a function of K alone, so a column shard equals its part of the whole."""
+    g = gen(770 + m + k)
+    base, x = torch.randn(64, k, generator=g).bfloat16().to(DEV), torch.randn(m, k, generator=g).bfloat16().to(DEV)
+    few, many = base.repeat(5, 1), base.repeat(513, 1)  # 64 and 128 k per stage, one to three blocks
+    _, narrow = lm_head_argmax(x, few, logits=True)
+    _, wide = lm_head_argmax(x, many, logits=True)
+    assert torch.equal(wide.view(m, -1, 64), narrow[:, None, :64].expand(m, 513, 64))
+    assert torch.equal(narrow.view(m, -1, 64), narrow[:, None, :64].expand(m, 5, 64))
+    if m > 16:  # up to there gate/up and partials choose their kernel by width
+        narrow, wide = (sk.linear_silu_mul(x, torch.cat([w, -w])) for w in (few, many))
+        assert torch.equal(wide.view(m, -1, 64), narrow[:, None, :64].expand(m, 513, 64))
+        narrow, wide = (sk.linear_partials(x, w) for w in (few, many))
+        assert torch.equal(wide.view(*narrow.shape[:2], -1, 64), narrow[:, :, None, :64].expand(-1, m, 513, 64))
+
+
 class _MLP(torch.nn.Module):
     def __init__(self, hidden, inner, g):
         super().__init__()
