@@ -52,6 +52,7 @@ struct StreamArgs {
   int32_t chunks;        // 64-wide k chunks per split
   int32_t tiles;         // n-tiles (gate/up: of 8 output columns) of the whole output
   int32_t groups;        // column groups: one workgroup each per split
+  int32_t block_tiles;   // tiles of a column block, at most
   int32_t splits;
   int32_t splits_major;  // 1: consecutive workgroups take the splits of one column group
 };
@@ -80,14 +81,15 @@ __device__ __forceinline__ void wait_loads() {
   static_assert(N >= 0 && N < 64, "vmcnt");
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
-// N = stages * PER, stages <= MAX.
+// All but the newest `stages` (at most MAX) stages of `per` (at most PER) loads each.
 template <int PER, int MAX>
-__device__ __forceinline__ void wait_stages(int stages) {
-  if constexpr (MAX == 0) {
+__device__ __forceinline__ void wait_stages(int per, int stages) {
+  if constexpr (MAX == 0 || PER == 0) {
     wait_loads<0>();
   } else {
-    if (stages >= MAX) wait_loads<MAX * PER>();
-    else wait_stages<PER, MAX - 1>(stages);
+    if (stages < MAX) wait_stages<PER, MAX - 1>(per, stages);
+    else if (per < PER) wait_stages<PER - 1, MAX>(per, stages);
+    else wait_loads<MAX * PER>();
   }
 }
 
@@ -124,7 +126,8 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
   const int64_t kbase = (int64_t)split * a.chunks * kChunk;
   const int stages = (a.chunks * kChunk + KW - 1) / KW;
   const bool ragged = !PHASED && KW > kChunk && (a.chunks & 1);  // last stage half filled
-  const int blocks = (t_hi - t_lo + NT - 1) / NT;
+  const int width = a.block_tiles;                 // <= NT: no loads for the rest
+  const int blocks = (t_hi - t_lo + width - 1) / width;
   const int total = blocks * stages;
 
   // Loads: tile i of a stage (NT of W, then MT of x) is loaded by the waves
@@ -155,6 +158,9 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
   constexpr int kParts = PHASED ? 4 : 1;
   const int per_part = stages / kParts;            // PHASED: K is a multiple of 1,024
   const int phase = PHASED ? (int)(((uint32_t)group * 0x9E3779B1u) >> 30) : 0;
+  // Loads of this wave per stage: its tiles of the block's W, and of x.
+  const int per_stage = (width > tg ? (width - tg + TG - 1) / TG : 0) +
+                        (MT > x0 ? (MT - x0 + TG - 1) / TG : 0);
   // Next stage to issue: stage is_in of part is_part of the block at is_tile.
   int is_tile = t_lo, is_part = 0, is_in = 0, is_stage = phase * per_part;
   auto issue = [&](int slot) {
@@ -166,9 +172,9 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
 #pragma unroll
     for (int c = 0; c < (NT + TG - 1) / TG; ++c) {
       const int i = tg + TG * c;
-      if (i < NT) {
+      if (i < width) {
         int t = is_tile + i;
-        if (t >= t_hi) t = is_tile;                // a block's missing tiles: its first again
+        if (t >= t_hi) t = is_tile;                // the last block's missing tiles: its first again
         const int64_t row = PAIRS ? (q < kTileLoads / 2 ? 0 : (int64_t)a.n - 8) + 8 * (int64_t)t +
                                         q * kLoadRows
                                   : (int64_t)kTile * t + q * kLoadRows;
@@ -185,7 +191,7 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
       is_in = 0;
       if (++is_part == kParts) {
         is_part = 0;
-        is_tile += NT;
+        is_tile += width;
       }
       is_stage = (is_part ^ phase) * per_part;
     }
@@ -242,7 +248,7 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
 #pragma unroll
     for (int i = 0; i < NTW; ++i) {
       const int t = tile0 + wn + NG * i;
-      const bool live = wn + NG * i < NT && t < t_hi;
+      const bool live = wn + NG * i < width && t < t_hi;
 #pragma unroll
       for (int j = 0; j < MTW; ++j) {
         const int m = kTile * (wm * MTW + j) + r;
@@ -292,12 +298,10 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
   for (int d = 0; d < S - 1; ++d)
     if (d < total) issue(d);
   int slot = 0, next = S - 1;
-  constexpr int kPer = kTiles / TG, kMore = kTiles % TG;  // loads per stage: kPer + (tg < kMore)
+  constexpr int kMostLoads = (NT + TG - 1) / TG + kXLoads;
   // Stage `it` of the sequence; `last`: the last one of its block.
   auto step = [&](int it, bool last) {
-    const int later = total - 1 - it;              // stages after this one, issued or not
-    if (tg < kMore) wait_stages<kPer + 1, S - 2>(later);
-    else wait_stages<kPer, S - 2>(later);
+    wait_stages<kMostLoads, S - 2>(per_stage, total - 1 - it);  // of the stages after this one
     __builtin_amdgcn_s_barrier();                  // stage `it` is whole; stage `it - 1` is read
     asm volatile("" ::: "memory");
     if (it + S - 1 < total) issue(next);
@@ -310,7 +314,7 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
   clear();
   int tile0 = t_lo;
   if constexpr (PHASED) {
-    for (int it = 0; it < total; tile0 += NT) {
+    for (int it = 0; it < total; tile0 += width) {
 #pragma unroll
       for (int part = 0; part < kParts; ++part) {
         for (int at = 0; at < per_part; ++at, ++it) step(it, false);
@@ -335,7 +339,7 @@ __global__ __launch_bounds__(kStreamBlock, 2) void stream_kernel(StreamArgs a) {
         store(tile0);
         clear();
         at = 0;
-        tile0 += NT;
+        tile0 += width;
       }
     }
   }
@@ -402,6 +406,7 @@ int launch_stream_as(const SkinnyArgs& s, int splits, hipStream_t stream) {
   constexpr int kMost = kMaxBlockTiles<MT, PHASED>;
   const int blocks = (most + kMost - 1) / kMost;
   const int need = (most + blocks - 1) / blocks;                 // tiles of a block
+  a.block_tiles = need;
   a.splits_major = splits > 1 && s.k >= s.n ? 1 : 0;
   const dim3 grid((unsigned)((int64_t)a.groups * splits));
 #define QF_STREAM(NT, KW)                                                              \
@@ -411,6 +416,9 @@ int launch_stream_as(const SkinnyArgs& s, int splits, hipStream_t stream) {
                        dim3(kStreamBlock), 0, stream, a);                              \
     return launch_status();                                                            \
   }
+  // A block loads the tiles it has, not its kernel's NT (a ladder, not every
+  // count): 89,344-column head at K = 2560, 22 tiles a workgroup as 2 x 11 on the
+  // 13-tile kernel, 64 rows 101 -> 95.8 us, 5 rows 79.2 -> 73.9.
   // Up to 8 tiles 128 k per stage (256-byte runs of each weight row), wider
   // blocks 64 k, so that three stages fit the LDS (Qwen3-4B qkv, 8 tiles, at
   // 32 and 64 rows 9.2 -> 8.7 and 10.9 -> 10.2 us with 128; gate/up, 5 tiles, at

@@ -29,7 +29,7 @@ def ints(shape, lo, hi, g):
 
 
 @pytest.mark.parametrize("m", [17, 32, 33, 48, 64])
-# 2 tiles | 257 shares of 256 | 24 tiles a workgroup (two blocks), K of 1, 3, 5 and 2 chunks a split
+# 2 tiles | 258 for 256 workgroups | 2 a workgroup | 2 or 3, K of 1, 3, 2 and 5 chunks a split
 @pytest.mark.parametrize("n,k,splits", [(32, 64, 1), (32, 192, 3), (4128, 192, 1), (6144, 128, 1),
                                         (2048, 320, 5), (416, 640, 2)])
 def test_partials(m, n, k, splits):
@@ -66,6 +66,50 @@ def test_lm_head(m, vocab, k):
     want = (x.double() @ w.double().T).float().to(torch.bfloat16)
     assert torch.equal(logits.cpu(), want)
     assert torch.equal(tokens.cpu(), want.float().argmax(-1))  # full of ties: the first maximum
+
+
+def device_ints(shape, most, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randint(-most, most + 1, shape, generator=g, device=DEV, dtype=torch.int8).bfloat16()
+
+
+@pytest.mark.parametrize("m", [17, 33, 64])
+# tiles a workgroup (as blocks, on the kernel for): 4 | 6 | 7 (8) | 9 (10) | 11 (13) | 15 (16) | 17 (19) | 20 (2 x 10) |
+# 12 splits x 23 (2 x 12 on 13), the last group shorter | 130 splits x 38 (2 x 19)
+@pytest.mark.parametrize("n,k,splits", [(16384, 320, 1), (24576, 448, 1), (28672, 320, 1), (36864, 320, 1), (45056, 448, 1),
+                                        (61440, 320, 1), (69632, 320, 1), (81920, 320, 1), (7456, 5376, 12),
+                                        (608, 41600, 130)])
+def test_partials_of_several_tiles_and_blocks(m, n, k, splits):
+    x, w = device_ints((m, k), 4, 780 + m), device_ints((n, k), 3, 781 + n)
+    got = torch.full((splits, m, n), float("nan"), device=DEV)
+    _lib.call("qf_linear_partials", x.data_ptr(), m, k, w.data_ptr(), n, splits, got.data_ptr(), _lib.stream(x.device))
+    for s in range(splits):
+        part = slice(s * (k // splits), (s + 1) * (k // splits))
+        assert torch.equal(got[s].double(), x[:, part].double() @ w[:, part].double().T), s
+
+
+@pytest.mark.parametrize("m", [17, 33, 64])
+# K in order: 3 ragged stages of 128 or 5 of 64 | in quarters: 8 of 128 or 16 of 64
+@pytest.mark.parametrize("k", [320, 1024])
+# 5 tiles a workgroup | 11 (13) | 18 (19; in quarters beyond 32 rows 2 x 9) | 20 (2 x 10), its last group shorter
+@pytest.mark.parametrize("n", [10240, 22528, 36864, 40928])
+def test_silu_mul_of_several_tiles_and_blocks(m, k, n):
+    x, w = device_ints((m, k), 2, 790 + m), device_ints((2 * n, k), 1, 791 + n)
+    got = sk.linear_silu_mul(x, w)
+    proj = (x.double() @ w.double().T).float().to(torch.bfloat16)
+    assert_bits_exact(got, O.silu_mul(bits(proj)), what=f"silu m={m} n={n} k={k}")
+
+
+@pytest.mark.parametrize("m", [5, 17, 33, 64])
+@pytest.mark.parametrize("k", [320, 1024])
+# 14 tiles a workgroup (16) | 39 (3 x 13)
+@pytest.mark.parametrize("vocab", [57344, 159760])
+def test_lm_head_of_several_tiles_and_blocks(m, k, vocab):
+    x, w = device_ints((m, k), 1, 795 + m), device_ints((vocab, k), 1, 796 + vocab)
+    tokens, logits = lm_head_argmax(x, w, logits=True)
+    want = (x.double() @ w.double().T).float().to(torch.bfloat16)
+    assert torch.equal(logits, want)
+    assert torch.equal(tokens.cpu(), want.float().cpu().argmax(-1))  # full of ties: the first maximum
 
 
 @pytest.mark.parametrize("m", [5, 33, 64])
