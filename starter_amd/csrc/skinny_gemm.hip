@@ -144,14 +144,14 @@ __device__ __forceinline__ void finish(const SkinnyArgs& a, f32x4 (&acc)[NT], ui
 #pragma unroll
     for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(dst + kTile * t) = acc[t];
   } else {
-    // Lanes of groups g = 0, 1 hold gate columns col0 + 4g .. +4; groups 2, 3
-    // the matching up columns, fetched across the wave's halves.  Each
-    // projection is a bf16 tensor in the reference; SiLU is rounded to bf16
-    // before the bf16 product.
+    // One tile: lanes of groups g = 0, 1 hold gate columns col0 + 4g .. +4;
+    // groups 2, 3 the matching up columns, fetched across the wave's halves.
+    // Two: a gate tile and its up tile.  Each projection is a bf16 tensor in
+    // the reference; SiLU is rounded to bf16 before the bf16 product.
     float up[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) up[i] = __shfl_xor(acc[0][i], 32);
-    if (g >= 2 || !row_ok) return;
+    for (int i = 0; i < 4; ++i) up[i] = NT == 1 ? __shfl_xor(acc[0][i], 32) : acc[NT - 1][i];
+    if ((NT == 1 && g >= 2) || !row_ok) return;
     float y[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -163,9 +163,10 @@ __device__ __forceinline__ void finish(const SkinnyArgs& a, f32x4 (&acc)[NT], ui
   }
 }
 
-// One m-tile of x (M <= 16) and NT n-tiles of W per workgroup (gate/up: one
-// tile of 8 gate rows over the matching 8 up rows, its two 8-row loads taken
-// from the two halves of the weight), every wave all of them over its own
+// One m-tile of x (M <= 16) and NT n-tiles of W per workgroup (gate/up: a gate
+// tile and the matching up tile, or one tile of 8 gate rows over the matching
+// 8 up rows, its two 8-row loads taken from the two halves of the weight),
+// every wave all of them over its own
 // chunks; D chunks in flight per wave; NTL = nontemporal weight loads; XS =
 // source of x (kXDirect, kXStaged, kXMerged, kXNormed).
 //
@@ -182,14 +183,15 @@ __device__ __forceinline__ void finish(const SkinnyArgs& a, f32x4 (&acc)[NT], ui
 // of qf_linear_partials / qf_linear_silu_mul on it.
 template <int NT, int D, int EPI, bool NTL, int XS, int PPT = 0>
 __global__ __launch_bounds__(kBlock) void skinny_kernel(SkinnyArgs a) {
-  constexpr bool HALF = EPI == kEpiSiluMul;
+  constexpr bool PAIRS = EPI == kEpiSiluMul;
+  constexpr bool HALF = PAIRS && NT == 1;
   constexpr bool XT = XS == kXStaged;
   constexpr bool XM = XS == kXMerged;
   constexpr bool XN = XS == kXNormed;
   constexpr bool XL = XM || XN;  // x read from the prologue's LDS slice
-  static_assert(!HALF || NT == 1, "gate/up: one half tile");
+  static_assert(!PAIRS || NT <= 2, "gate/up: a half tile or a pair");
   static_assert(!XN || (kBlock == QF_ROW_GROUPS && PPT >= 1), "normed x: one sum per thread and row");
-  constexpr int kColW = HALF ? kTile / 2 : kTile * NT;  // output columns
+  constexpr int kColW = PAIRS ? kTile / 2 * NT : kTile * NT;  // output columns
   constexpr int kStageTiles = NT + (XT ? 1 : 0);
   constexpr int kStageBytes = kWaves * kStageTiles * kTileLds;
   constexpr int kHandoffBytes = (kWaves - 1) * NT * kWave * 16;
@@ -212,7 +214,7 @@ __global__ __launch_bounds__(kBlock) void skinny_kernel(SkinnyArgs a) {
   const uint16_t* wp[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
-    wp[t] = a.w + (int64_t)(col0 + kTile * t + lane / 8) * a.k + kbase + 8 * (lane % 8);
+    wp[t] = a.w + (int64_t)(col0 + (PAIRS ? a.n : kTile) * t + lane / 8) * a.k + kbase + 8 * (lane % 8);
   const int64_t wstep = HALF ? (int64_t)a.n * a.k : (int64_t)kRowsPerLoad * a.k;
   // Lanes of x rows beyond M read row 0 instead: the MFMA keeps every
   // output column separate, and those columns are never stored.
@@ -470,7 +472,7 @@ dim3 skinny_grid(SkinnyArgs& a, int64_t grid_x, int splits) {
 
 template <int NT, int D, int EPI, bool NTL, int XS, int PPT = 0>
 int launch(const SkinnyArgs& args, int splits, hipStream_t s, size_t dyn_lds = 0) {
-  constexpr int kColsPerBlock = EPI == kEpiSiluMul ? kTile / 2 : kTile * NT;
+  constexpr int kColsPerBlock = EPI == kEpiSiluMul ? kTile / 2 * NT : kTile * NT;
   SkinnyArgs a = args;
   const dim3 grid = skinny_grid(a, a.n / kColsPerBlock, splits);
   hipLaunchKernelGGL((skinny_kernel<NT, D, EPI, NTL, XS, PPT>), grid, dim3(kBlock), dyn_lds, s, a);
@@ -508,17 +510,33 @@ int dispatch_partials(const SkinnyArgs& a, int splits, hipStream_t s) {
   return launch<1, 2, kEpiPartials, true, kXStaged>(a, splits, s);
 }
 
-// Gate/up + SiLU: all of K per workgroup.  Up to 4 rows one tile of 8 gate
-// over 8 up rows per workgroup (1,216 workgroups for Qwen3-4B: 10% faster
-// than a gate and an up tile per wave, whose 608 larger workgroups leave the
-// stream's end unbalanced; the addition order of the normalising form, whose
-// bits these rows share); beyond, one weight stream per CU (Qwen3-4B against
-// such tiles with x staged per wave at 5 and 16 rows, 20.1 -> 18.7 and 21.7 ->
-// 18.9 us, and against 128-column workgroups at 17 and 64, 23.6 -> 19.4 and
-// 30.6 -> 23.9).
+// Where gate/up at 9..16 rows is a weight stream: K beyond 2,048 and at least
+// three tiles of 8 columns per stream workgroup, four up to 12 rows (K = 2560,
+// tiles here -> stream: 9,728 columns at 9 rows 19.2 -> 18.2 us, 12 20.0 -> 18.2, 16
+// 21.5 -> 18.3; 5,120 columns 12.4 -> 12.9, 13.0 -> 12.9, 15.1 -> 13.0; K = 4096, 8,192
+// columns 25.4 -> 23.8, 25.2 -> 24.0, 26.6 -> 24.0).  Less leaves the stream's
+// one workgroup per CU too little to hide its fill and serial stages behind:
+// two tiles at 9 rows 10.0 -> 11.8, K = 1024 with 3,072 columns at 16 rows 5.5 -> 7.0;
+// K = 2048 is even, and up to 8 rows nothing gains.
+bool wide_gate_up(const SkinnyArgs& a) {
+  const int32_t most = (a.n / (kTile / 2) + kCUs - 1) / kCUs;  // tiles of a stream workgroup
+  return a.k > 2048 && a.m > 8 && most >= (a.m > 12 ? 3 : 4);
+}
+
+// Gate/up + SiLU: all of K per workgroup.  Up to 12 rows one tile of 8 gate
+// over 8 up rows per workgroup (1,216 workgroups for Qwen3-4B: 10% faster at
+// 1-4 rows than a gate and an up tile per wave, whose 608 larger workgroups
+// leave the stream's end unbalanced; the addition order of the normalising
+// form, whose bits these rows share); 13..16 rows the tile pair, whose x reads
+// weigh half (same bits; 11,008 columns at K = 2560 25.2 -> 22.4 us at 16, but 2,048 9.3
+// against 7.6); beyond, and where wide_gate_up says so, one weight
+// stream per CU (Qwen3-4B against 128-column workgroups at 17 and 64 rows,
+// 23.6 -> 19.4 and 30.6 -> 23.9).
 int dispatch_silu(const SkinnyArgs& a, hipStream_t s) {
+  if (a.m > kTile || wide_gate_up(a)) return stream_silu(a, s);
   if (a.m <= 4) return launch<1, 4, kEpiSiluMul, true, kXDirect>(a, 1, s);
-  return stream_silu(a, s);
+  if (a.m <= 12) return launch<1, 4, kEpiSiluMul, true, kXStaged>(a, 1, s);
+  return launch<2, 4, kEpiSiluMul, true, kXStaged>(a, 1, s);
 }
 
 // Final argmax over a row's candidates: one workgroup per row, each thread

@@ -88,6 +88,26 @@ def test_partials_of_several_tiles_and_blocks(m, n, k, splits):
         assert torch.equal(got[s].double(), x[:, part].double() @ w[:, part].double().T), s
 
 
+@pytest.mark.parametrize("k,n", [(64, 32), (320, 96), (1024, 2080), (2112, 4096), (2048, 8224)])
+def test_gate_up_rows_up_to_16_share_their_bits(k, n):
+    """Below the stream's widths a row's result does not depend on the rows beside it."""
+    g = torch.Generator(device=DEV).manual_seed(785 + n)
+    x, w = (torch.randn(rows, k, generator=g, device=DEV).bfloat16() for rows in (16, 2 * n))
+    whole = sk.linear_silu_mul(x, w)
+    for m in (1, 4, 5, 8, 9, 12, 13):
+        assert torch.equal(sk.linear_silu_mul(x[:m].contiguous(), w), whole[:m]), m
+
+
+@pytest.mark.parametrize("m", [5, 9, 12, 13, 16])
+# one tile a stream workgroup | two, and three | three, and four, at the K on both sides of the rule
+@pytest.mark.parametrize("n,k", [(96, 2112), (4096, 2112), (4128, 2112), (6144, 2112), (6176, 2112), (4128, 3072), (6176, 2048)])
+def test_gate_up_on_both_sides_of_the_streams_rule(m, n, k):
+    x, w = device_ints((m, k), 2, 786 + m), device_ints((2 * n, k), 1, 787 + n)
+    got = sk.linear_silu_mul(x, w)
+    proj = (x.double() @ w.double().T).float().to(torch.bfloat16)
+    assert_bits_exact(got, O.silu_mul(bits(proj)), what=f"silu m={m} n={n} k={k}")
+
+
 @pytest.mark.parametrize("m", [17, 33, 64])
 # K in order: 3 ragged stages of 128 or 5 of 64 | in quarters: 8 of 128 or 16 of 64
 @pytest.mark.parametrize("k", [320, 1024])
