@@ -426,6 +426,146 @@ __global__ __launch_bounds__(kBlock) void skinny_kernel(SkinnyArgs a) {
   finish<NT, EPI>(a, acc, lds, lane, wave, col0, split);
 }
 
+// f32 partials at 17..64 rows of short K ranges, which end before the weight
+// stream's ring is full (dispatch_partials).  Small workgroups of four
+// waves, NT n-tiles each over the same chunks, in any number per CU; the workgroup
+// stages each x chunk once, cooperatively and coalesced, in a shared LDS ring
+// of two buffers (one barrier per step: a buffer is rewritten only after every
+// wave has passed the barrier that follows its last read), W still goes
+// through each wave's own staging tile, D chunks in flight.  One wave and one
+// chain of additions per output, so the bits are the stream's.  Waves whose
+// tiles lie past N stream row 0 and store nothing.
+template <int MT, int NT>
+__global__ __launch_bounds__(kBlock) void shared_x_kernel(SkinnyArgs a) {
+  constexpr int D = 4;
+  constexpr int kRows = kTile * MT;                    // staged x rows (M padded)
+  constexpr int kPieces = kRows * (kChunk * 2 / 16);   // 16-byte pieces per chunk
+  constexpr int XL = (kPieces + kBlock - 1) / kBlock;  // x loads per thread per chunk
+  constexpr int kXBytes = kRows * kLdsRow;             // one ring buffer
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kXBytes + kWaves * NT * kTileLds];
+
+  const int tid = threadIdx.x;
+  const int lane = tid % kWave;
+  const int wave = tid / kWave;
+  const int r = lane % kTile;
+  const int g = lane / kTile;
+  const int col0 = ((a.splits_major ? blockIdx.y : blockIdx.x) * kWaves + wave) * (kTile * NT);
+  const bool live = col0 < a.n;
+  const int split = a.splits_major ? blockIdx.x : blockIdx.y;
+  const int64_t kbase = (int64_t)split * a.chunks * kChunk;
+
+  const uint16_t* wp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    // N is a multiple of 32, so of a wave's two tiles both or none are past it.
+    const int row = live ? col0 + kTile * t : 0;
+    wp[t] = a.w + (int64_t)(row + lane / 8) * a.k + kbase + 8 * (lane % 8);
+  }
+  const int64_t wstep = (int64_t)kRowsPerLoad * a.k;
+  // Piece p = tid + 256 i of a chunk: x row p / 8 (row 0 stands in for rows
+  // past M), 16 bytes at column 8 * (p % 8).
+  const uint16_t* xp[XL];
+  int xoff[XL];
+  bool xon[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int p = tid + kBlock * i;
+    xon[i] = p < kPieces;
+    const int row = xon[i] ? p / 8 : 0;
+    xp[i] = a.x + (int64_t)(row < a.m ? row : 0) * a.k + kbase + 8 * (p % 8);
+    xoff[i] = lds_off(row, p % 8);
+  }
+  uint8_t* stage = lds + 2 * kXBytes + wave * NT * kTileLds;
+  const int wr_off[2] = {lds_off(lane / 8, lane % 8), lds_off(lane / 8 + kRowsPerLoad, lane % 8)};
+  const int rd_off[2] = {lds_off(r, g), lds_off(r, g + 4)};
+
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  uint4 wv[D][NT][2], xv[D][XL];
+  auto issue = [&](int d, int j) {
+    const int64_t off = (int64_t)j * kChunk;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) wv[d][t][i] = load16<true>(wp[t] + off + i * wstep);
+#pragma unroll
+    for (int i = 0; i < XL; ++i) xv[d][i] = xon[i] ? load16<false>(xp[i] + off) : make_uint4(0, 0, 0, 0);
+  };
+  auto consume = [&](int d, int j) {
+    uint8_t* xb = lds + (j & 1) * kXBytes;
+#pragma unroll
+    for (int i = 0; i < XL; ++i)
+      if (xon[i]) *reinterpret_cast<uint4*>(xb + xoff[i]) = xv[d][i];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<uint4*>(stage + t * kTileLds + wr_off[i]) = wv[d][t][i];
+    __syncthreads();
+    uint4 fw[NT][2], fx[MT][2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        fw[t][s] = *reinterpret_cast<const uint4*>(stage + t * kTileLds + rd_off[s]);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        fx[mt][s] = *reinterpret_cast<const uint4*>(xb + mt * kTileLds + rd_off[s]);
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[t][mt] = mfma(fw[t][s], fx[mt][s], acc[t][mt]);
+  };
+
+  // The software pipeline of skinny_kernel; every wave takes all chunks.
+  if (a.chunks >= D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) issue(d, d);
+    int j = 0;
+    for (; j + 2 * D <= a.chunks; j += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        consume(d, j + d);
+        issue(d, j + d + D);
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      consume(d, j + d);
+      if (j + d + D < a.chunks) issue(d, j + d + D);
+    }
+    j += D;
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (j + d < a.chunks) consume(d, j + d);
+  } else {
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (d < a.chunks) issue(d, d);
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (d < a.chunks) consume(d, d);
+  }
+
+  if (!live) return;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int m = kTile * mt + r;
+    if (m >= a.m) continue;
+    float* dst = a.partials + ((int64_t)split * a.m + m) * a.n + col0 + 4 * g;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(dst + kTile * t) = acc[t][mt];
+  }
+}
+
 // ---- launch plans -----------------------------------------------------------
 
 int shape_status(int64_t rows, int64_t k, int64_t n) {
@@ -496,15 +636,51 @@ int launch_normed(const SkinnyArgs& a, int splits, hipStream_t s) {
   }
 }
 
+// Two n-tiles per wave (128 columns per workgroup, half the x re-reads of one)
+// while that leaves at most one workgroup per CU, else one.
+template <int MT>
+int launch_shared_x(const SkinnyArgs& args, int splits, hipStream_t s) {
+  SkinnyArgs a = args;
+  const int64_t wide = ((int64_t)a.n + 8 * kTile - 1) / (8 * kTile);
+  if (wide * splits <= kCUs) {
+    const dim3 grid = skinny_grid(a, wide, splits);
+    hipLaunchKernelGGL((shared_x_kernel<MT, 2>), grid, dim3(kBlock), 0, s, a);
+  } else {
+    const dim3 grid = skinny_grid(a, ((int64_t)a.n + 4 * kTile - 1) / (4 * kTile), splits);
+    hipLaunchKernelGGL((shared_x_kernel<MT, 1>), grid, dim3(kBlock), 0, s, a);
+  }
+  return launch_status();
+}
+
+// Where those workgroups are ahead of the weight stream (linear_partials and
+// the add + norm behind it at N = 2560, here against the stream): K ranges of up
+// to 4 chunks once a stream workgroup has more than 10 tiles, since a range
+// ends before the ring is full and many splits leave few column groups, so
+// CUs without one (K = 8896, 139 splits and 139 workgroups: 34.1 against 40.5 us at 17 rows,
+// 50.0 against 62.0 at 64; K = 5696, 89 splits: 25.5, 28.8 and 35.3, 38.3); with fewer
+// tiles the stream is (N = 1024, K = 2880 at 64 rows 10.6, 9.3).  At 8 chunks, by the
+// block: exactly 8 tiles up to 48 rows (K = 6144 at 48 rows 15.1, 15.5) and
+// over 11 up to 32 (K = 9728 at 17 rows 16.8, 17.2); otherwise the two are even or the stream
+// is ahead (K = 9728 at 64 rows 23.0, 22.4).
+bool short_ranges(const SkinnyArgs& a, int splits) {
+  const int32_t tiles = a.n / kTile, groups = stream_groups(tiles, splits);
+  const int32_t most = (tiles + groups - 1) / groups;  // of a stream workgroup
+  if (a.chunks < 5) return most > 10;
+  return a.chunks == 8 && ((a.m <= 3 * kTile && most == 8) || (a.m <= 2 * kTile && most > 11));
+}
+
 // Tile plans (measured): up to 4 rows of x arrive as one broadcast line per
 // load, so x goes straight into MFMA layout; up to 16 x is loaded like W and
 // transposed through LDS by each wave (the addition order of
 // qf_linear_partials_merged, whose bits these rows share); beyond 16 rows one
-// weight stream per CU (Qwen3-4B at 64 rows against 128-column workgroups
-// staging x per 64 k: qkv 10.6 -> 10.2 us, o_proj 8.4 -> 7.9, down 15.1 ->
-// 13.6; at 17 rows 8.4 -> 8.4, 7.1 -> 6.7, 11.5 -> 11.6).
+// weight stream per CU, or small workgroups (short_ranges).
 int dispatch_partials(const SkinnyArgs& a, int splits, hipStream_t s) {
-  if (a.m > kTile) return stream_partials(a, splits, s);
+  if (a.m > kTile) {
+    if (!short_ranges(a, splits)) return stream_partials(a, splits, s);
+    if (a.m <= 2 * kTile) return launch_shared_x<2>(a, splits, s);
+    if (a.m <= 3 * kTile) return launch_shared_x<3>(a, splits, s);
+    return launch_shared_x<4>(a, splits, s);
+  }
   if (a.m <= 4) return launch<1, 2, kEpiPartials, true, kXDirect>(a, splits, s);
   if (a.n / kTile >= 256) return launch<2, 2, kEpiPartials, true, kXStaged>(a, splits, s);
   return launch<1, 2, kEpiPartials, true, kXStaged>(a, splits, s);

@@ -73,12 +73,16 @@ def device_ints(shape, most, seed):
     return torch.randint(-most, most + 1, shape, generator=g, device=DEV, dtype=torch.int8).bfloat16()
 
 
-@pytest.mark.parametrize("m", [17, 33, 64])
+@pytest.mark.parametrize("m", [17, 32, 33, 48, 64])
 # tiles a workgroup (as blocks, on the kernel for): 4 | 6 | 7 (8) | 9 (10) | 11 (13) | 15 (16) | 17 (19) | 20 (2 x 10) |
 # 12 splits x 23 (2 x 12 on 13), the last group shorter | 130 splits x 38 (2 x 19)
 @pytest.mark.parametrize("n,k,splits", [(16384, 320, 1), (24576, 448, 1), (28672, 320, 1), (36864, 320, 1), (45056, 448, 1),
                                         (61440, 320, 1), (69632, 320, 1), (81920, 320, 1), (7456, 5376, 12),
-                                        (608, 41600, 130)])
+                                        (608, 41600, 130),
+                                        # small workgroups: one chunk a split, two, four, columns past the last tile
+                                        (2560, 5056, 79), (608, 8896, 139), (640, 12800, 100), (352, 33024, 129),
+                                        # and at 8 chunks: blocks of 8 tiles up to 48 rows, of 13 up to 32
+                                        (2560, 6144, 12), (2592, 6144, 12), (2560, 9728, 19)])
 def test_partials_of_several_tiles_and_blocks(m, n, k, splits):
     x, w = device_ints((m, k), 4, 780 + m), device_ints((n, k), 3, 781 + n)
     got = torch.full((splits, m, n), float("nan"), device=DEV)
