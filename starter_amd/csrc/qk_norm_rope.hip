@@ -179,8 +179,11 @@ constexpr int kUnitsPerWave = 2;
 // halves the chain (1 x 17 tokens 3.3 -> 2.6 us, 1 x 128 3.5 -> 2.8, 1 x 512
 // 5.7 -> 5.4; 1 x 1024 7.4 with two units, 8.0 with one).  Below the streaming
 // size workgroups are one wave, which spread over more CUs (1 x 1024 7.8 ->
-// 7.3 us, 16 x 128 11.6 -> 11.3); streaming calls keep four (4 x 2048 34.9
-// against 36.3).
+// 7.3 us, 16 x 128 11.6 -> 11.3; 5 units a token, 1 x 1400 9.4 -> 7.8);
+// streaming calls keep four (4 x 2048 34.9 against 36.3), and so do tokens of an
+// even number of waves whose last has one unit: consecutive workgroups go to
+// the 8 XCDs in turn, so half or a quarter of the XCDs would get all the
+// short waves (3 units a token, 1 x 2048: 8.3 us, with four waves 6.8).
 constexpr uint64_t kSmallUnits = 12 * kCUs;
 constexpr int kRowLanes = 8;  // lanes per head row in the unit kernel
 
@@ -461,7 +464,8 @@ extern "C" int qf_prefill_qkv(const void* qkv, int64_t batch, int64_t length, in
     else if (stream && full) QF_UNITS(true, true, kUnitsPerWave, kBlock, wide);
     else if (stream) QF_UNITS(true, false, kUnitsPerWave, kBlock, wide);
     else if (full) QF_UNITS(false, true, kUnitsPerWave, kWave, narrow);
-    else QF_UNITS(false, false, kUnitsPerWave, kWave, narrow);
+    else if (per_token % 2 != 0) QF_UNITS(false, false, kUnitsPerWave, kWave, narrow);
+    else QF_UNITS(false, false, kUnitsPerWave, kBlock, wide);
 #undef QF_UNITS
     return launch_status();
   }

@@ -1,6 +1,6 @@
 """Prompt kernels on both sides of their dispatch rules: the attention's
 workgroup forms, and the Q/K/V kernel's units per wave (one up to 3,072 units of
-8 head rows, two beyond)."""
+8 head rows, two beyond, in workgroups of one wave or four)."""
 
 from __future__ import annotations
 
@@ -55,7 +55,7 @@ def test_attention_forms_at_eight_heads_per_kv_head(batch, length):
 
 
 @pytest.mark.parametrize("batch,length,nq,nk", [(1, 1, 32, 8), (3, 5, 16, 8), (1, 512, 32, 8), (1, 513, 32, 8),
-                                                (7, 110, 16, 8), (1, 1100, 8, 8)])
+                                                (7, 110, 16, 8), (1, 1100, 8, 8), (1, 700, 24, 8), (3, 300, 40, 8)])
 def test_qkv_units_per_wave(batch, length, nq, nk):
     g = gen(820 + length)
     capacity = length + 2
