@@ -599,7 +599,11 @@ int launch_prefill_as(PrefillArgs a, bool ordered, hipStream_t s) {
 // quarter of its).  Of those, prompts that its positions per workgroup fit
 // badly take the mid form, half as wide: under four wide blocks of positions,
 // or up to six blocks with the last at most half full; the shortest of all
-// take 16 positions.
+// take 16 positions.  But at G = 4 not where the wide grid is exactly one
+// workgroup per CU, which all end together (32 over 8 heads, mid / wide: 8 x 250
+// 17.9 / 16.4 us, 8 x 200 15.9 / 15.4; one pair more, 9 x 250 17.8 / 21.9), and
+// six blocks only beyond 9/8 of that (16 over 4, 12 x 340 20.9 / 20.2, 13 x 340
+// 18.8 / 20.9).
 template <int G>
 int launch_prefill(PrefillArgs a, hipStream_t s) {
   constexpr int QB = Split<G, kWide>::QB;
@@ -608,7 +612,11 @@ int launch_prefill(PrefillArgs a, hipStream_t s) {
     return launch_prefill_as<G, kNarrow>(a, false, s);
   if constexpr (G >= 4) {
     if (G == 4 && a.length <= 16) return launch_prefill_as<G, kNarrow>(a, false, s);
-    if (a.length < 4 * QB || (wide <= 6 && tail <= QB / 2)) return launch_prefill_as<G, kMid>(a, true, s);
+    const int64_t grid = wide * a.pairs;
+    const bool even = G == 4 && a.length > 2 * QB && grid == kCUs;
+    const int most = G == 4 && 8 * grid <= 9 * (int64_t)kCUs ? 5 : 6;
+    if (!even && (a.length < 4 * QB || (wide <= most && tail <= QB / 2)))
+      return launch_prefill_as<G, kMid>(a, true, s);
   }
   return launch_prefill_as<G, kWide>(a, true, s);
 }

@@ -54,6 +54,21 @@ def test_attention_forms_at_eight_heads_per_kv_head(batch, length):
     check_attention(batch, length, 16, 2)
 
 
+# at 32 over 8 heads: 16 | 17 positions; exactly one wide workgroup per CU and more; six blocks up to 9/8 of
+# that and beyond; over six.  16 over 8: four per CU.  16 over 2: 32 positions a block
+@pytest.mark.parametrize("batch,length,hq,hk", [(33, 16, 32, 8), (33, 17, 32, 8), (8, 250, 32, 8), (9, 250, 32, 8), (8, 257, 32, 8),
+                                                (6, 352, 32, 8), (7, 352, 32, 8), (9, 353, 32, 8), (9, 400, 32, 8),
+                                                (32, 200, 16, 8), (64, 127, 16, 2), (64, 144, 16, 2), (64, 145, 16, 2)])
+def test_attention_forms_give_the_same_bits(batch, length, hq, hk):
+    """A sequence alone runs the narrow form, in a batch the one its grid asks for."""
+    g = torch.Generator(device=DEV).manual_seed(810 + length)
+    q, k, v = (torch.randn(1, *shape, 128, generator=g, device=DEV).bfloat16()
+               for shape in ((length, hq), (hk, length), (hk, length)))
+    alone = prefill_attention(q, k, v, length, 128 ** -0.5)
+    many = prefill_attention(*(t.expand(batch, -1, -1, -1).contiguous() for t in (q, k, v)), length, 128 ** -0.5)
+    assert torch.equal(many, alone.expand_as(many))
+
+
 @pytest.mark.parametrize("batch,length,nq,nk", [(1, 1, 32, 8), (3, 5, 16, 8), (1, 512, 32, 8), (1, 513, 32, 8),
                                                 (7, 110, 16, 8), (1, 1100, 8, 8), (1, 700, 24, 8), (3, 300, 40, 8)])
 def test_qkv_units_per_wave(batch, length, nq, nk):
