@@ -114,7 +114,7 @@ struct PrefillArgs {
 // kNarrow: one tile per wave (two workgroups per CU where LDS allows) on the
 // single-wave pipeline: the most workgroups and the shortest chain per key
 // block, for grids that do not fill the chip.  kMid and kWide: 8 waves on the
-// ping-pong schedule, one and two tiles per wave (G = 2: one, 64 positions).
+// ping-pong schedule, one and two tiles per wave (G = 2: one, 64 positions; G = 1: 4 waves, one tile each, for all).
 // All forms give the same bits.  Measured (Qwen3-4B heads, us, narrow / mid /
 // wide): 1 x 512 13.4 / - / 18.7, 1 x 1024 23.2 / 36.9 / 30.0, 8 x 128 8.3 / 8.4 /
 // 10.8, 16 x 128 13.4 / 12.7 / 12.9, 64 x 17 10.5 / 8.3 / 14.3, 64 x 64 20.8 /
@@ -127,7 +127,7 @@ struct PrefillArgs {
 // 13.5 -> 11.0), no ping-pong at G = 2 (4 x 2048 117.9 -> 93.9).
 constexpr int kNarrow = 0, kMid = 1, kWide = 2;
 template <int G, int FORM> struct Split;
-template <int FORM> struct Split<1, FORM> { static constexpr int QB = 64, TPW = 1, W = 4; };
+template <> struct Split<1, kWide> { static constexpr int QB = 64, TPW = 1, W = 4; };
 template <> struct Split<2, kNarrow> { static constexpr int QB = 32, TPW = 1, W = 4; };
 template <> struct Split<2, kWide> { static constexpr int QB = 64, TPW = 1, W = 8; };
 template <> struct Split<4, kNarrow> { static constexpr int QB = 16, TPW = 1, W = 4; };
@@ -608,8 +608,12 @@ template <int G>
 int launch_prefill(PrefillArgs a, hipStream_t s) {
   constexpr int QB = Split<G, kWide>::QB;
   const int64_t wide = (a.length + QB - 1) / QB, tail = a.length - (wide - 1) * QB;
-  if (wide * a.pairs < (G == 2 ? 4 : 1) * (int64_t)kCUs)
+  const bool narrow = wide * a.pairs < (G == 2 ? 4 : 1) * (int64_t)kCUs;
+  if constexpr (G == 1) {
+    return launch_prefill_as<G, kWide>(a, !narrow, s);  // one shape for all grids
+  } else if (narrow) {
     return launch_prefill_as<G, kNarrow>(a, false, s);
+  }
   if constexpr (G >= 4) {
     if (G == 4 && a.length <= 16) return launch_prefill_as<G, kNarrow>(a, false, s);
     const int64_t grid = wide * a.pairs;
