@@ -4,7 +4,8 @@
   epsilon and calls ``kernels.rmsnorm.rms_norm``.
 * ``PackedMLP`` - engine/mlp.py:8-21: one packed ``[2I, H]`` gate/up weight;
   on CUDA bf16 the activation is the fused ``silu_mul`` kernel on the packed
-  projection (up to 64 rows one launch for both, ``linear_silu_mul``), elsewhere it is the reference module's own ``act_fn(gate) * up``.
+  projection (up to 64 rows one launch for both, ``linear_silu_mul``),
+  elsewhere it is the reference module's own ``act_fn(gate) * up``.
 * ``DecodeQKNormRoPE`` - engine/qk_norm_rope.py:10-71: a ``Qwen3Attention``
   whose single-token decode forward runs the per-head Q/K RMSNorm and the
   rotary embedding as one ``kernels.qk_norm_rope`` launch; every other call
@@ -20,6 +21,8 @@ import copy
 
 import torch
 from torch import nn
+from torch.overrides import has_torch_function
+from torch.utils._python_dispatch import is_in_torch_dispatch_mode
 from torch.nn import functional as F
 
 from transformers.modeling_utils import ALL_ATTENTION_FUNCTIONS
@@ -49,6 +52,13 @@ def _is_silu(act) -> bool:
     return isinstance(act, nn.SiLU) or type(act).__name__ in ("SiLUActivation", "SiLU")
 
 
+def _plain(*tensors) -> bool:
+    """Ordinary tensors outside any torch function or dispatch mode: a kernel
+    may take their memory in place of a torch call that nobody else is to see."""
+    return (all(type(t) in (torch.Tensor, nn.Parameter) for t in tensors)
+            and not has_torch_function(tensors) and not is_in_torch_dispatch_mode())
+
+
 class PackedMLP(nn.Module):
     @torch.no_grad()
     def __init__(self, reference):
@@ -66,9 +76,13 @@ class PackedMLP(nn.Module):
         not apply.  The library's product reads the same weight at under half
         its rate there, then writes and re-reads the projections (this module
         at the Qwen3-4B widths, 1 / 21 / 64 rows: 66.5 -> 38.1 us, 53.6 -> 39.5,
-        62.7 -> 52.3).  64 rows are what the stream kernel's x tiles hold."""
+        62.7 -> 52.3; ahead at 1-64 rows of every width measured, least at K =
+        1024, 2,240 columns: 21.2 -> 18.9 at 12 rows).  64 rows are what the
+        stream kernel's x tiles hold.  A tensor subclass (a quantised weight)
+        or a mode that watches torch calls keeps the torch product."""
         if (not x.is_cuda or x.dtype != torch.bfloat16 or x.ndim < 1 or torch.is_autocast_enabled("cuda")
-                or not 1 <= x.numel() // max(x.shape[-1], 1) <= MAX_ROWS or not _is_silu(self.act_fn)):
+                or not 1 <= x.numel() // max(x.shape[-1], 1) <= MAX_ROWS or not _is_silu(self.act_fn)
+                or not _plain(x, self.gate_up_weight)):
             return None
         rows = x.reshape(-1, x.shape[-1])
         if not supports(rows, self.gate_up_weight, pairs=True):

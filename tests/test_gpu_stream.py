@@ -200,3 +200,47 @@ def test_packed_mlp_on_both_sides_of_its_row_rule(shape, inner, form):
         want = module.down_proj(torch.nn.functional.silu(gate) * up)
     assert got.shape == want.shape and got.dtype == want.dtype
     torch.testing.assert_close(got.float(), want.float(), rtol=0.02, atol=0.02 * float(want.float().abs().max()) if want.numel() else 0)
+
+
+class _Scaled(torch.Tensor):
+    """A weight without memory of its own, as quantised ones are: bf16(values * 0.5) when a product asks."""
+
+    @staticmethod
+    def __new__(cls, values):
+        return torch.Tensor._make_wrapper_subclass(cls, values.shape, dtype=torch.bfloat16, device=values.device)
+
+    def __init__(self, values):
+        self.values = values
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        if func is torch.ops.aten.detach.default:
+            return cls(args[0].values)
+        return func(*[a.values * 0.5 if isinstance(a, _Scaled) else a for a in args], **(kwargs or {}))
+
+
+@torch.no_grad()
+def test_packed_mlp_leaves_subclassed_weights_and_watched_calls_to_torch():
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Seen(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.ops = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    g = gen(765)
+    module = modules.PackedMLP(_MLP(256, 320, g).cuda().bfloat16())
+    x = torch.randn(3, 256, generator=g).cuda().bfloat16()
+    with Seen() as seen:
+        module(x)
+    assert sum("mm" in op or "linear" in op for op in seen.ops) == 2, seen.ops  # both products
+    weight = module.gate_up_weight
+    halved = torch.nn.Parameter(weight * 0.5, requires_grad=False)
+    module.gate_up_weight = halved
+    want = module(x)
+    module.gate_up_weight = torch.nn.Parameter(_Scaled(weight.data), requires_grad=False)
+    torch.testing.assert_close(module(x).float(), want.float(), rtol=0.02, atol=0.02 * float(want.float().abs().max()))
