@@ -37,7 +37,8 @@ OBJ_DIR = PACKAGE / "_build"
 LIBRARY = PACKAGE / "kernels" / "libqwen_fused.so"
 PHASES_LIBRARY = PACKAGE / "kernels" / "libqwen_fused_phases.so"
 PHASES_SOURCE = "decode_attention.hip"
-HOST_CALLS = PACKAGE / "kernels" / "_host_calls.so"
+# one interpreter's ABI, by its name
+HOST_CALLS = PACKAGE / "kernels" / f"_host_calls{sysconfig.get_config_var('EXT_SUFFIX')}"
 HOST_SOURCE = "host_calls.cpp"
 SOURCES = ("rmsnorm.hip", "silu_mul.hip", "qk_norm_rope.hip", "embedding.hip", "skinny_gemm.hip",
            "stream_gemm.hip", "decode_attention.hip", "prefill_attention.hip", "row_gemv.hip")
@@ -81,9 +82,12 @@ def _cxx() -> str:
 
 def _host_flags() -> list[str]:
     """Flags of the Python extension: torch's and HIP's headers (HIP's want to
-    know the platform when no HIP compiler says it)."""
+    know the platform when no HIP compiler says it), and the torch build they
+    belong to, which the extension compares with the one that imports it."""
+    from torch import version
     include = _torch_dir() / "include"
     return ["-O2", "-fPIC", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f'-DQF_TORCH_BUILD="{version.__version__} {version.git_version}"',
             "-I", str(ROOT / "include"), "-isystem", str(include),
             "-isystem", str(include / "torch" / "csrc" / "api" / "include"),
             "-isystem", str(Path(hipcc()).resolve().parents[1] / "include"),

@@ -4,7 +4,8 @@
 // host in Python: operand checks attribute by attribute, the output
 // allocation, the stream lookup and a ctypes call of 8-23 converted
 // arguments.  Each function here does the same for the ordinary case - plain
-// contiguous tensors of one GPU - in 3-5 us, and returns NotImplemented, having
+// contiguous tensors of one GPU - in about half of that (rms_norm [8, 2560] 10.3 ->
+// 5.8 us a call, its launch included), and returns NotImplemented, having
 // done nothing, for every other one: the Python wrapper then runs its own
 // checks and raises or launches as before.  Nothing is decided here that the
 // wrapper decides differently, so what is refused, and how, stays there.
@@ -428,4 +429,26 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", "Native forms of the
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host_calls() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host_calls() {
+  // Everything above reads torch's C++ objects as the headers of one torch
+  // build lay them out, so the import fails under any other (the file's name
+  // carries the interpreter's ABI); the wrappers then go their own way.
+  PyObject* torch = PyImport_ImportModule("torch.version");
+  PyObject* version = torch ? PyObject_GetAttrString(torch, "__version__") : nullptr;
+  PyObject* revision = version ? PyObject_GetAttrString(torch, "git_version") : nullptr;
+  PyObject* running = revision ? PyUnicode_FromFormat("%S %S", version, revision) : nullptr;
+  PyObject* made = nullptr;
+  if (running && PyUnicode_CompareWithASCIIString(running, QF_TORCH_BUILD) == 0) {
+    made = PyModule_Create(&module);
+  } else if (running) {
+    PyErr_Format(PyExc_ImportError, "built for torch %s, this is %U", QF_TORCH_BUILD, running);
+  } else {
+    PyErr_Clear();
+    PyErr_Format(PyExc_ImportError, "built for torch %s, this one names no version", QF_TORCH_BUILD);
+  }
+  Py_XDECREF(running);
+  Py_XDECREF(revision);
+  Py_XDECREF(version);
+  Py_XDECREF(torch);
+  return made;
+}
