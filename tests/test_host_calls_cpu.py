@@ -1,6 +1,6 @@
-"""The native wrappers' module where it cannot serve: another torch build, or a
-file that does not load.  The kernels' own library and the Python path do not
-depend on it."""
+"""The native wrappers' module where it cannot serve: another torch build, a
+file that does not load, a machine without a C++ compiler.  The kernels' own
+library and the Python path do not depend on it."""
 
 from __future__ import annotations
 
@@ -12,6 +12,7 @@ import torch
 
 from conftest import ROOT
 
+from starter_amd import build
 from starter_amd.kernels import _lib
 from starter_amd.kernels.rmsnorm import rms_norm
 
@@ -44,3 +45,26 @@ print(native, any("built for torch" in str(w.message) for w in seen))
 """
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, check=True)
     assert out.stdout.split()[-2:] == (["False", "True"] if attribute else ["True", "False"])
+
+
+@pytest.mark.parametrize("broken", ["compiler", "torch", None])
+def test_the_library_is_linked_without_it(broken, tmp_path, monkeypatch, capsys):
+    """Commands are recorded, not run: each leaves its output file."""
+    def run(cmd, verbose):
+        if broken == "compiler" and cmd[0] == "g++":
+            raise FileNotFoundError("g++")
+        (tmp_path / cmd[cmd.index("-o") + 1]).write_text("")
+
+    monkeypatch.setattr(build, "_run", run)
+    monkeypatch.setattr(build, "_cxx", lambda: "g++")
+    monkeypatch.setattr(build, "hipcc", lambda: "/opt/rocm/bin/hipcc")
+    if broken == "torch":
+        monkeypatch.setattr(build.importlib.util, "find_spec", lambda name: None)
+    for name, file in (("LIBRARY", "lib.so"), ("PHASES_LIBRARY", "phases.so"), ("HOST_CALLS", "host.so")):
+        monkeypatch.setattr(build, name, tmp_path / file)
+    monkeypatch.setattr(build, "OBJ_DIR", tmp_path / "objects")
+    (tmp_path / "host.so").write_text("an older build's")
+    assert build.build() == tmp_path / "lib.so"
+    assert (tmp_path / "lib.so").exists() and (tmp_path / "phases.so").exists()
+    assert (tmp_path / "host.so").exists() == (broken is None)
+    assert ("is not built" in capsys.readouterr().err) == (broken is not None)
