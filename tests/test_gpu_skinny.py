@@ -82,7 +82,7 @@ def test_partials_integer_exact_every_path(m):
 
 
 @pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 12, 13, 16, 17, 33, 64])  # 12 | 13: half tile | tile pairs
-@pytest.mark.parametrize("n", [64, 96])  # 96: the last workgroup has waves past N
+@pytest.mark.parametrize("n", [64, 96])  # even and odd numbers of 32 columns
 def test_silu_mul_integer_exact_every_path(m, n):
     g = gen(80 + m + n)
     k = 640

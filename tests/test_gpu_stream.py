@@ -185,7 +185,7 @@ class _MLP(torch.nn.Module):
 @pytest.mark.parametrize("inner", [320, 96])  # 96: not whole column pairs, the library's product
 @pytest.mark.parametrize("form", ["plain", "strided", "autocast"])
 @torch.no_grad()
-def test_packed_mlp_on_both_sides_of_its_row_rule(shape, inner, form):
+def test_packed_mlp_on_both_sides_of_its_row_rule(shape, inner, form, monkeypatch):
     """The module on decode-sized inputs against the projections and activation in sequence: within
     the f32 accumulation of a projection, which moves single bf16 values by one rounding."""
     g = gen(760 + inner)
@@ -193,8 +193,11 @@ def test_packed_mlp_on_both_sides_of_its_row_rule(shape, inner, form):
     x = torch.randn(shape, generator=g).cuda().bfloat16()
     if form == "strided":
         x = torch.stack([x, x], -1)[..., 0]
+    taken = []
+    monkeypatch.setattr(modules, "linear_silu_mul", lambda *args: taken.append(args) or sk.linear_silu_mul(*args))
     with torch.autocast("cuda", dtype=torch.float16, enabled=form == "autocast"):
         got = module(x)
+        assert len(taken) == (1 <= x.shape[:-1].numel() <= 64 and inner == 320 and form != "autocast")
         projected = torch.nn.functional.linear(x, module.gate_up_weight)
         gate, up = projected.chunk(2, -1)
         want = module.down_proj(torch.nn.functional.silu(gate) * up)
