@@ -66,8 +66,8 @@ inline int32_t stream_groups(int32_t tiles, int splits) {
   return fill < tiles ? fill : tiles;
 }
 
-// The 17..64-row projections (stream_gemm.hip): x, w, partials / out, k, m, n
-// and chunks set, checked by the caller.
+// The weight streams (stream_gemm.hip; partials at 17..64 rows, the others at
+// any): x, w, partials / out, k, m, n and chunks set, checked by the caller.
 int stream_partials(const SkinnyArgs& a, int splits, hipStream_t s);
 int stream_silu(const SkinnyArgs& a, hipStream_t s);
 int stream_argmax(const SkinnyArgs& a, hipStream_t s);

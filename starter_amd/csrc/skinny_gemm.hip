@@ -28,7 +28,9 @@
 // take interleaved chunks of that range, so together they read consecutive
 // bytes of every row, and reduce their f32 tiles through LDS in wave order.
 // Rows of x beyond M are never stored.  This kernel serves up to 16 rows of
-// x; more (and gate/up and the LM head from 5 rows) go to stream_gemm.hip.
+// x, except the LM head from 5 rows and wide gate/up from 9, which like most
+// calls beyond 16 rows go to stream_gemm.hip; short K ranges beyond 16 rows
+// stay here (shared_x_kernel).
 //
 // Two epilogues, as in the reference:
 //   * qf_linear_partials: the workgroup's f32 tile is split `split`'s partial
@@ -580,9 +582,11 @@ int shape_status(int64_t rows, int64_t k, int64_t n) {
 // 3072 workgroups of 16 columns (~12 per CU), and the partials (written here,
 // read by the consumer) small: splits * min(M, 16) <= K / 32, at most 8 (o_proj
 // takes the same time at 8 and 16 splits, and its consumer, one workgroup per
-// row, reads half the bytes).  Beyond 16 rows: K ranges of at most 512 (eight
-// chunks) per workgroup, the fewest splits that give them (Qwen3-4B: qkv 5,
-// o_proj 8, down 19 splits).
+// row, reads half the bytes).  Beyond 16 rows: equal K ranges of at most 512
+// (eight chunks), the fewest splits that give them (Qwen3-4B: qkv 5, o_proj 8,
+// down 19 splits).  A chunk count without a divisor near an eighth of itself
+// gets short ranges, down to one chunk each where it is prime (K = 8896: 139
+// splits, whose partials outweigh the weight at 48 rows).
 int plan_splits(int64_t rows, int64_t k, int64_t n) {
   const int64_t chunks = k / kChunk;
   const int64_t mrows = rows < kTile ? rows : kTile;
@@ -783,11 +787,15 @@ __global__ __launch_bounds__(kFinThreads) void argmax_finalize_kernel(const uint
   }
 }
 
-// LM head plans (measured on the Qwen3-4B head, 151936 x 2560): up to 4 rows
-// (x as broadcast lines) one 16-column tile per workgroup, the most
+// LM head plans (measured on the Qwen3-4B head, 151936 x 2560, logits kept): up
+// to 4 rows (x as broadcast lines) one 16-column tile per workgroup, the most
 // workgroups; beyond, one weight stream per CU, whose wide column blocks
-// re-read x twice per CU instead of once per 128 columns (8 rows 129.2 ->
-// 125.9 us, 16 134.8 -> 124.9, 32 143.3 -> 130.5, 64 159.6 -> 140.7).
+// re-read x twice per CU instead of once per 32 columns (5 rows 122.9 ->
+// 120.5 us, 8 127.7 -> 121.2) or per 128 (16 132.2 -> 125.0, 32 148.7 -> 133, 64
+// 178 -> 152).  Other widths from 32,000 columns at 5-8 rows: ahead of
+// the 32-column workgroups by 1, 6 and 2% on average at K = 1024, 2048 and 2560,
+// at worst 8% behind (122,112 columns, K = 2048); up to 4,096 columns, at
+// most one tile a CU, up to 3 us behind.
 constexpr int kArgmaxTileRows = 4;
 int dispatch_argmax(const SkinnyArgs& a, hipStream_t s) {
   if (a.m <= kArgmaxTileRows) return launch<1, 4, kEpiArgmax, true, kXDirect>(a, 1, s);

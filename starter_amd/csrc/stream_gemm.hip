@@ -1,16 +1,20 @@
-// Decode projections y = x @ W^T for 17..64 rows of x as one weight stream per
-// compute unit (engine/kernels/skinny_gemm.py:28-121 is the reference).
+// Decode projections y = x @ W^T as one weight stream per compute unit: partials at
+// 17..64 rows of x, gate/up from 9 and the LM head from 5 (skinny_gemm.hip
+// says which calls; engine/kernels/skinny_gemm.py:28-121 is the reference).
 //
 // What bounds it: HBM, the weight read once; at these row counts x (up to 64 x
 // K) comes from L2 for every column block and weighs as much as the weights
 // do in the CU's own traffic.  So one 8-wave workgroup per CU takes an equal
 // share of the output columns (the fewest, widest column blocks that fill the
 // chip, so x is re-read the least), and everything moves by
-// global_load_lds_dwordx4 straight into an LDS ring of 128-wide k stages:
-// no registers hold loads in flight, and up to ~110 KB per CU are, whatever
-// the waves are doing.  One barrier per stage; a stage's loads are waited for
-// by count (vmcnt, S - 2 stages stay in flight over the wait).  A workgroup
-// whose columns need several blocks runs them through one continuous ring.
+// global_load_lds_dwordx4 straight into an LDS ring of three stages, 128 k wide
+// for blocks of up to 8 tiles and 64 beyond: no registers hold loads in
+// flight, and up to two stages (96 KB) per CU are, whatever the waves are
+// doing.  One barrier per stage; a stage's loads are waited for by count
+// (vmcnt, S - 2 stages stay in flight over the wait).  A workgroup whose
+// columns need several blocks runs them through one continuous ring.  K ranges
+// of a few stages do not fill it (64-row qkv and o_proj, four stages: 42 reads
+// in flight per CU where the LM head holds 95).
 //
 //   A operand = 16 rows of W (one n-tile), B operand = 16 rows of x (one
 //   m-tile), 32 k per v_mfma_f32_16x16x32_bf16; lane l's result is
@@ -19,9 +23,13 @@
 //   (tile t to group t % (8 / MG)); every output has one wave and one chain
 //   of additions, so no reduction between waves is needed.
 //
-// A ring tile is 16 rows of 256 bytes; 16-byte piece p of row r sits at piece
-// p ^ r, so the 16 lanes of a fragment read touch all 64 banks once.  The DMA
-// writes linearly, so the lanes fetch permuted pieces of the same 256 bytes.
+// A ring tile is 16 rows of 256 or 128 bytes; 16-byte piece p of row r sits at
+// piece p ^ swizzle(r), so the 16 lanes of a fragment read touch all 64 banks
+// once.  The DMA writes linearly, so the lanes fetch permuted pieces of a
+// row's own bytes.
+//
+// Every call's order of additions is a function of K and its split count
+// (launch_stream), not of the columns or of the rows beside a row.
 //
 // Gate/up tiles hold 8 gate rows over the matching 8 up rows: the SiLU
 // epilogue is local to the wave.
