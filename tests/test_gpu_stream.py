@@ -182,7 +182,7 @@ class _MLP(torch.nn.Module):
 
 
 @pytest.mark.parametrize("shape", [(1, 256), (2, 3, 256), (64, 256), (65, 256), (1, 0, 256)])
-@pytest.mark.parametrize("inner", [320, 96])  # 96: not whole column pairs, the library's product
+@pytest.mark.parametrize("inner", [320, 96, 80])  # 80: not whole column pairs, the library's product
 @pytest.mark.parametrize("form", ["plain", "strided", "autocast"])
 @torch.no_grad()
 def test_packed_mlp_on_both_sides_of_its_row_rule(shape, inner, form, monkeypatch):
@@ -197,7 +197,7 @@ def test_packed_mlp_on_both_sides_of_its_row_rule(shape, inner, form, monkeypatc
     monkeypatch.setattr(modules, "linear_silu_mul", lambda *args: taken.append(args) or sk.linear_silu_mul(*args))
     with torch.autocast("cuda", dtype=torch.float16, enabled=form == "autocast"):
         got = module(x)
-        assert len(taken) == (1 <= x.shape[:-1].numel() <= 64 and inner == 320 and form != "autocast")
+        assert len(taken) == (1 <= x.shape[:-1].numel() <= 64 and inner != 80 and form == "plain")
         projected = torch.nn.functional.linear(x, module.gate_up_weight)
         gate, up = projected.chunk(2, -1)
         want = module.down_proj(torch.nn.functional.silu(gate) * up)
