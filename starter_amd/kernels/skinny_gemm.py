@@ -67,9 +67,9 @@ def split_count(n, k, rows=1):
     """K splits of ``linear_partials`` for x [rows, k] @ W[n, k].T.
 
     Each split covers an equal run of whole 64-wide k chunks, so the count
-    divides k / 64: a power of two up to 16 rows; beyond, K ranges of about
-    512 per workgroup (5, 8 and 19 splits on the Qwen3-4B shapes).  The plan
-    lives in the library (qf_linear_splits) so C callers get the same one;
+    divides k / 64: a power of two up to 16 rows; beyond, K ranges of at most
+    512 (5, 8 and 19 splits on the Qwen3-4B shapes; one per chunk where k / 64
+    is prime).  The plan lives in the library (qf_linear_splits) so C callers get the same one;
     compare engine/kernels/skinny_gemm.py:86-91, which ignores rows.
     """
     status = _lib.lib().qf_linear_splits(int(rows), int(k), int(n))
